@@ -1055,34 +1055,36 @@ extern "C" int mgpu_ad_step(mgpu_ad *ad, const mgpu_ad_args *a, double *prop) {
 // one device take turns.
 namespace {
 struct SolverScratch {
-    double *W = nullptr;            // forward-sweep W, Size-shaped
+    double *W = nullptr;            // forward-sweep W (mgpu_thomas3d: W and G)
     double *st[5] = {};             // host mode: D, E, F, TI, res on the device
     int32_t *wp = nullptr;          // host mode: WaterPoints3D on the device
     unsigned long long *piv = nullptr;
-    long cap = 0;                   // cells each array holds
+    long cap = 0;                   // cells each staging array holds
+    long wcap = 0;                  // doubles W holds
 };
 constexpr int MAX_DEVICES = 64;
 std::mutex g_scr_mu;
 SolverScratch g_scr[MAX_DEVICES];
 
-// The calling device's scratch with room for n cells (host: also the
-// staging arrays), or null (rc set).
-SolverScratch *solver_scratch(long n, bool host, int &rc) {
+// The calling device's scratch with nw doubles in W (host: also staging
+// arrays of n cells), or null (rc set).
+SolverScratch *solver_scratch(long n, long nw, bool host, int &rc) {
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) { mgpu_set_error("hipGetDevice", e); rc = MGPU_ERR_HIP; return nullptr; }
     if (dev < 0 || dev >= MAX_DEVICES) { rc = MGPU_ERR_BADARG; return nullptr; }
     SolverScratch &q = g_scr[dev];
-    if (q.cap < n) {
+    if (q.wcap < nw) {
         dfree(q.W);
+        q.wcap = 0;
+        if (dalloc(&q.W, nw)) { rc = MGPU_ERR_NOMEM; return nullptr; }
+        q.wcap = nw;
+    }
+    if (host && (!q.st[0] || q.cap < n)) {
+        int r = 0;
         for (double *&a : q.st) dfree(a);
         dfree(q.wp);
-        q.cap = 0;
-        if (dalloc(&q.W, n)) { rc = MGPU_ERR_NOMEM; return nullptr; }
         q.cap = n;
-    }
-    if (host && !q.st[0]) {
-        int r = 0;
         for (double *&a : q.st) r |= dalloc(&a, q.cap);
         r |= dalloc(&q.wp, q.cap);
         if (r) {
@@ -1108,7 +1110,7 @@ extern "C" int mgpu_thomasz(const mgpu_size3d *size, const mgpu_size3d *worksize
     const size_t b3 = sizeof(double) * (size_t)n3;
     hipStream_t s = (hipStream_t)stream;
     std::lock_guard<std::mutex> lock(g_scr_mu);
-    SolverScratch *q = solver_scratch(n3, !dev, rc);
+    SolverScratch *q = solver_scratch(n3, n3, !dev, rc);
     if (!q) return rc;
     hipError_t e = hipSuccess;
     if (dev) {
@@ -1210,7 +1212,9 @@ extern "C" int mgpu_thomas3d(const mgpu_size3d *size, int32_t IJmin, int32_t IJm
     hipStream_t s = (hipStream_t)stream;
     int rc = 0;
     std::lock_guard<std::mutex> lock(g_scr_mu);
-    SolverScratch *q = solver_scratch(n3, !dev, rc);
+    const long nw = thomas3d_scratch((long)(IJmax - IJmin + 1) * (Kmax - Kmin + 1),
+                                     JImax - JImin + 2);
+    SolverScratch *q = solver_scratch(n3, nw, !dev, rc);
     if (!q) return rc;
     double *dD = q->st[0], *dE = q->st[1], *dF = q->st[2], *dT = q->st[3], *dR = q->st[4];
     unsigned long long npiv = 0;

@@ -382,10 +382,12 @@ int launch_copy_lines(const Dims &d, int axis, const double *src, double *dst,
 // along k, j and i (the ghost rows of the drop-in's TI record).
 int launch_land_fill(const Dims &d, const uint8_t *mask, double *dst, hipStream_t s);
 // THOMAS_3D lines (di 0: along j, IJ = i; di 1: along i, IJ = j) on arrays
-// spanning sz; bounds already checked.  pivots counts lines with a zero pivot.
+// spanning sz; bounds already checked.  pivots counts lines with a zero pivot;
+// scr holds thomas3d_scratch(lines, rows) doubles.
+long thomas3d_scratch(long nl, int nrow);
 int launch_thomas3d(const mgpu_size3d &sz, int IJmin, int IJmax, int JImin, int JImax, int Kmin,
                     int Kmax, int di, const double *D, const double *E, const double *F,
-                    const double *TI, double *res, double *Wscr, unsigned long long *pivots,
+                    const double *TI, double *res, double *scr, unsigned long long *pivots,
                     hipStream_t s);
 int launch_thomasz(const Dims &d, const double *D, const double *E, const double *F,
                    const double *TI, const int32_t *wp, double *res, double *Wscr,

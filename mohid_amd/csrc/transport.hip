@@ -211,80 +211,6 @@ int launch_slot_fields(const Dims &d, const SlotColumns &S, const double *Qz, co
     return MGPU_SUCCESS;
 }
 
-namespace {
-// THOMAS_3D_i0_j1_NewType / _i1_j0_NewType (MF:3756-3870) on explicit
-// arrays: one lane per (IJ, K) line; the line's rows are sJI apart from
-// row JImin at base0 + IJ * sIJ + K * sK.  W goes to Wscr, G to res, which
-// the back substitution then overwrites with the solution.
-__global__ void thomas3d_kernel(long base0, long sIJ, long sJI, long sK, int nIJ, long nl,
-                                int nrow, const double *__restrict__ D,
-                                const double *__restrict__ E, const double *__restrict__ F,
-                                const double *__restrict__ TI, double *__restrict__ res,
-                                double *__restrict__ Wscr, unsigned long long *__restrict__ pivots) {
-    const long line = blockIdx.x * (long)blockDim.x + threadIdx.x;
-    if (line >= nl) return;
-    const long b = base0 + (line % nIJ) * sIJ + (line / nIJ) * sK;
-    double Wm = -F[b] / E[b];
-    double Gm = TI[b] / E[b];
-    Wscr[b] = Wm;
-    res[b] = Gm;
-    bool pivot = false;
-    for (int r = 1; r < nrow; ++r) {
-        const long x = b + r * sJI;
-        const double Dr = D[x];
-        const double aux = E[x] + Dr * Wm;
-        double W = 0.0, G = 0.0;
-        if (fabs(aux) > 0.0) {
-            W = -F[x] / aux;
-            G = (TI[x] - Dr * Gm) / aux;
-        } else {
-            pivot = true;
-        }
-        Wscr[x] = W;
-        res[x] = G;
-        Wm = W;
-        Gm = G;
-    }
-    double xs = Gm;
-    for (int r = nrow - 2; r >= 0; --r) {
-        const long x = b + r * sJI;
-        xs = Wscr[x] * xs + res[x];
-        res[x] = xs;
-    }
-    if (pivot) atomicAdd(pivots, 1ull);
-}
-}  // namespace
-
-int launch_thomas3d(const mgpu_size3d &sz, int IJmin, int IJmax, int JImin, int JImax, int Kmin,
-                    int Kmax, int di, const double *D, const double *E, const double *F,
-                    const double *TI, double *res, double *Wscr, unsigned long long *pivots,
-                    hipStream_t s) {
-    const long nI = sz.IUB - sz.ILB + 1, nJ = sz.JUB - sz.JLB + 1;
-    const long sj = nI, sk = nI * nJ;
-    const long sIJ = di == 0 ? 1 : sj, sJI = di == 0 ? sj : 1;
-    const long base0 = di == 0
-        ? (IJmin - sz.ILB) + (JImin - sz.JLB) * sj + (Kmin - sz.KLB) * sk
-        : (JImin - sz.ILB) + (IJmin - sz.JLB) * sj + (Kmin - sz.KLB) * sk;
-    const int nIJ = IJmax - IJmin + 1;
-    const long nl = (long)nIJ * (Kmax - Kmin + 1);
-    const int nrow = JImax - JImin + 2;
-    if (nl <= 0 || nrow <= 0) return MGPU_SUCCESS;
-    hipLaunchKernelGGL(thomas3d_kernel, dim3((unsigned)((nl + 255) / 256)), dim3(256), 0, s,
-                       base0, sIJ, sJI, sk, nIJ, nl, nrow, D, E, F, TI, res, Wscr, pivots);
-    HIPCHK(hipGetLastError());
-    return MGPU_SUCCESS;
-}
-
-int launch_thomasz(const Dims &d, const double *D, const double *E, const double *F,
-                   const double *TI, const int32_t *wp, double *res, double *Wscr,
-                   hipStream_t s) {
-    const int ni = d.wIUB - d.wILB + 1, nj = d.wJUB - d.wJLB + 1;
-    dim3 b(64, 4), g((ni + 63) / 64, (nj + 3) / 4);
-    hipLaunchKernelGGL(thomasz_kernel, g, b, 0, s, d, D, E, F, TI, wp, res, Wscr);
-    HIPCHK(hipGetLastError());
-    return MGPU_SUCCESS;
-}
-
 // ---------------------------------------------------------------------------
 // One tracer between a Fortran array and an interleaved buffer.
 namespace {

@@ -1094,46 +1094,6 @@ vertical_kernel(Dims d, StepScalars sc, SharedFields f, TracerSet ts, double *__
 }
 
 // ---------------------------------------------------------------------------
-// Stand-alone THOMASZ_NewType2 (MF:4026-4123) on caller-held D/E/F/TI.
-__global__ void thomasz_kernel(Dims d, const double *__restrict__ D,
-                               const double *__restrict__ E, const double *__restrict__ F,
-                               const double *__restrict__ TI, const int32_t *__restrict__ wp,
-                               double *__restrict__ res, double *__restrict__ Wscr) {
-    const int i = d.wILB + blockIdx.x * blockDim.x + threadIdx.x;
-    const int j = d.wJLB + blockIdx.y * blockDim.y + threadIdx.y;
-    if (i > d.wIUB || j > d.wJUB) return;
-    const int KLB = d.wKLB, KUB = d.wKUB;
-    if (wp[d.idx(i, j, KUB)] != 1) return;
-    // row 1 (MF:4087-4088 index the first row with the literal 1)
-    long x = d.idx(i, j, 1);
-    double Wm = -F[x] / E[x];
-    double Gm = TI[x] / E[x];
-    Wscr[x] = Wm;
-    res[x] = Gm;
-    for (int k = KLB + 1; k <= KUB + 1; ++k) {
-        x = d.idx(i, j, k);
-        const double Dk = D[x];
-        const double aux = E[x] + Dk * Wm;
-        double W = 0.0, G = 0.0;
-        if (fabs(aux) > 0.0) {
-            W = -F[x] / aux;
-            G = (TI[x] - Dk * Gm) / aux;
-        }
-        Wscr[x] = W;
-        res[x] = G;
-        Wm = W;
-        Gm = G;
-    }
-    double x1 = Gm;
-    for (int k = KUB; k >= KLB; --k) {
-        x = d.idx(i, j, k);
-        x1 = Wscr[x] * x1 + res[x];
-        res[x] = x1;
-    }
-}
-
-
-// ---------------------------------------------------------------------------
 // Lane variant.  One lane per (cell, tracer) builds the explicit right-hand
 // side, one lane per (column, tracer) solves the column; lanes run over
 // compact lists of the cells and columns the reference solves, in memory

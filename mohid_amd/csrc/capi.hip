@@ -240,12 +240,14 @@ struct DevDerived {
     long ncells = 0, ncols = 0, nhrows = 0;
     // [0] THOMASZ zero pivots, [1] bad-method flag, [2] mask flags, [3] THOMAS_3D zero pivots
     unsigned long long *counters = nullptr;
-    int alloc(const Dims &d) {
+    // cell_list: also the list of solved rows, for launches of several tracers
+    int alloc(const Dims &d, bool cell_list) {
         const long n3 = d.n3(), nt = tile_count(d), nK = d.KUB - d.KLB + 1;
         const long nIw = d.wIUB - d.wILB + 1, nJw = d.wJUB - d.wJLB + 1,
                    nKw = d.wKUB - d.wKLB + 1;
         int rc = 0;
-        rc |= dalloc(&rowcnt, nJw * nKw); rc |= dalloc(&cells, nIw * nJw * nKw);
+        rc |= dalloc(&rowcnt, nJw * nKw);
+        if (cell_list) rc |= dalloc(&cells, nIw * nJw * nKw);
         rc |= dalloc(&cols, nIw * nJw); rc |= dalloc(&totals, 3);
         rc |= dalloc(&mask, n3); rc |= dalloc(&kstart, d.n2());
         rc |= dalloc(&cu, n3); rc |= dalloc(&cv, n3); rc |= dalloc(&cw, n3);
@@ -287,7 +289,7 @@ struct DevDerived {
         unsigned long long n[3];
         HIPCHK(hipMemcpyAsync(n, totals, sizeof(n), hipMemcpyDeviceToHost, s));
         HIPCHK(hipStreamSynchronize(s));
-        ncells = (long)n[0];
+        ncells = cells ? (long)n[0] : 0;
         ncols = (long)n[1];
         nhrows = hlines ? (long)n[2] : 0;
         return MGPU_SUCCESS;
@@ -511,7 +513,7 @@ extern "C" int mgpu_ad_create(const mgpu_size3d *size, const mgpu_size3d *worksi
     }
     const long n3 = ad->d.n3();
     rc = ad->geom.alloc(ad->d);
-    if (!rc) rc = ad->der.alloc(ad->d);
+    if (!rc) rc = ad->der.alloc(ad->d, false);
     if (!rc) rc = dalloc(&ad->prop, n3);
     if (!rc) rc = dalloc(&ad->out, n3);
     const long scr = n3 > blocked_scratch_len(ad->d, 1) ? n3 : blocked_scratch_len(ad->d, 1);
@@ -1458,7 +1460,7 @@ extern "C" int mgpu_transport_create(const mgpu_size3d *size, const mgpu_size3d 
     }
     const long n3 = t->d.n3();
     rc = t->geom.alloc(t->d);
-    if (!rc) rc = t->der.alloc(t->d);
+    if (!rc) rc = t->der.alloc(t->d, opts->ntracers > 1);
     const long nT = (long)opts->ntracers;
     // scratch: tile-blocked (split) or laid out like the state (lanes, fused)
     long scr = blocked_scratch_len(t->d, opts->ntracers);

@@ -73,8 +73,21 @@ __device__ __forceinline__ double clamp_min_value(double dc) {
     return dc;
 }
 
+// One instruction each for fmin and fmax; a NaN ratio gives 2 here as it does
+// with the reference's comparisons (only the sign of a zero may differ).
 __device__ __forceinline__ double superbee_theta(double r) {
-    return dmax(dmax(0.0, dmin(1.0, 2.0 * r)), dmin(r, 2.0));
+    return fmax(fmax(0.0, fmin(1.0, 2.0 * r)), fmin(r, 2.0));
+}
+
+// Theta of the other limiters that take the ratio alone (MF:10702-10894); `bad`
+// is set for an id the reference stops on.
+__device__ __forceinline__ double limiter_theta(int tvd, double rr, int &bad) {
+    if (tvd == LIM_MINMOD) return dmax(0.0, dmin(1.0, rr));
+    if (tvd == LIM_VANLEER) return (rr < 0.0) ? 0.0 : 2.0 * rr / (1.0 + rr);
+    if (tvd == LIM_MUSCL) return dmax(0.0, dmin(dmin(2.0, 2.0 * rr), (1.0 + rr) / 2.0));
+    if (tvd == LIM_SUPERBEE) return superbee_theta(rr);
+    bad = 1;
+    return 0.0;
 }
 
 // ComputeAdvectionFace for every method/limiter; `bad` is set where the

@@ -225,7 +225,8 @@ int launch_prep_faces(const Dims &d, const double *visc, const double *diffv,
 //     kernel (W over TI in Wb, G in Gb); Wb and Gb tile-blocked,
 //     blocked_scratch_len(d, n) doubles each (chunk c at offset
 //     blocked_scratch_len(d, first tracer of c)).
-//   variant MGPU_KERNEL_LANES: lane-per-(cell, tracer) explicit kernel and
+//   variant MGPU_KERNEL_LANES: lane-per-(cell, tracer) explicit kernel (a
+//     launch of one tracer: tiles of columns, one level each) and
 //     lane-per-(column, tracer) column kernel over `lists`; Wb and Gb are
 //     laid out like the state (n * Size doubles each, tracer t of cell x at
 //     [x * stride + t]).  With lanes.mixed the column kernel is the
@@ -261,15 +262,16 @@ struct SlotColumns {
 
 // Compact lists of the lane variant (device arrays, host counts).
 struct SolveLists {
-    const uint32_t *cells = nullptr;   // Size index of every solved row, memory order
+    const uint32_t *cells = nullptr;   // Size index of every solved row, memory order (null:
+                                       // not built; a launch of one tracer needs none)
     const uint32_t *cols = nullptr;    // Size index (level 0) of every solved column
     const uint32_t *hrows = nullptr;   // WorkSize cells without M_HID (implicit line rows)
     long ncells = 0, ncols = 0, nhrows = 0;
     SlotColumns slot;                  // the depth-ordered walk's columns (batched transport)
 };
 // Builds the lists from the packed masks and kstart; totals[0..2] receive
-// the counts (device memory; the caller copies them back); hrows may be null
-// (not built).  rowcnt holds (WorkSize J extent) x (WorkSize K extent)
+// the counts (device memory; the caller copies them back); cells and hrows
+// may be null (not built).  rowcnt holds (WorkSize J extent) x (WorkSize K extent)
 // counters.
 int launch_build_lists(const Dims &d, const uint8_t *mask, const int32_t *kstart,
                        uint32_t *rowcnt, uint32_t *cells, uint32_t *cols, uint32_t *hrows,

@@ -66,14 +66,17 @@ int launch_build_lists(const Dims &d, const uint8_t *mask, const int32_t *kstart
     if (d.n3() >= (1L << 32)) return MGPU_ERR_UNSUPPORTED;   // list entries are 32-bit
     const int nj = d.wJUB - d.wJLB + 1, nk = d.wKUB - d.wKLB + 1;
     // cells: rows (j, k); columns: rows j
-    hipLaunchKernelGGL(list_count_kernel, dim3(nj, nk), dim3(256), 0, s, d, mask, kstart, 0,
-                       rowcnt);
-    HIPCHK(hipGetLastError());
-    hipLaunchKernelGGL(list_scan_kernel, dim3(1), dim3(1024), 0, s, rowcnt, (long)nj * nk, totals);
-    HIPCHK(hipGetLastError());
-    hipLaunchKernelGGL(list_write_kernel, dim3(nj, nk), dim3(256), 0, s, d, mask, kstart, 0,
-                       rowcnt, cells);
-    HIPCHK(hipGetLastError());
+    if (cells) {
+        hipLaunchKernelGGL(list_count_kernel, dim3(nj, nk), dim3(256), 0, s, d, mask, kstart, 0,
+                           rowcnt);
+        HIPCHK(hipGetLastError());
+        hipLaunchKernelGGL(list_scan_kernel, dim3(1), dim3(1024), 0, s, rowcnt, (long)nj * nk,
+                           totals);
+        HIPCHK(hipGetLastError());
+        hipLaunchKernelGGL(list_write_kernel, dim3(nj, nk), dim3(256), 0, s, d, mask, kstart, 0,
+                           rowcnt, cells);
+        HIPCHK(hipGetLastError());
+    }
     hipLaunchKernelGGL(list_count_kernel, dim3(nj, 1), dim3(256), 0, s, d, mask, kstart, 1,
                        rowcnt);
     HIPCHK(hipGetLastError());
@@ -109,7 +112,7 @@ int launch_transport(const TransportLaunch &L, const Dims &d, const StepScalars 
     if (L.variant != MGPU_KERNEL_FUSED && L.variant != MGPU_KERNEL_SPLIT &&
         L.variant != MGPU_KERNEL_LANES)
         return MGPU_ERR_BADARG;
-    if (L.variant != MGPU_KERNEL_SPLIT && (!L.lists.cells || !L.lists.cols)) return MGPU_ERR_BADARG;
+    if (L.variant != MGPU_KERNEL_SPLIT && !L.lists.cols) return MGPU_ERR_BADARG;
     if (!L.Wb || !L.Gb || !L.P || !L.out) return MGPU_ERR_BADARG;
     if (sc.impH >= 0) {
         // the line solves are built on the lane variant's state-shaped scratch

@@ -11,11 +11,14 @@
 //   prep_faces      face conductances Kh*A/dx (U, V faces) and
 //                   Kz*DUX*DVY/DZZ (W faces), AD:2364-2675 + AD:1514-1619;
 //   explicit        the explicit right-hand side TI of every solved cell
-//                   (AD:3966-4021, 4368-4953, 5156-5365): by default one lane
-//                   per (cell, group of tracers) over the cell list, the
-//                   cell's whole cross stencil loaded before any arithmetic
-//                   (explicit_lane_kernel); the tile variant computes each
-//                   face once into LDS (explicit_kernel);
+//                   (AD:3966-4021, 4368-4953, 5156-5365): by default, for
+//                   several tracers, one lane per (cell, group of tracers)
+//                   over the cell list, the cell's whole cross stencil loaded
+//                   before any arithmetic (explicit_lane_kernel), and for one
+//                   tracer each face computed once into LDS, over the faces
+//                   and cells a block finds active (explicit_tile_kernel); the
+//                   tile variant does that over sorted lists
+//                   (explicit_kernel);
 //   column          one lane per (water column, group of tracers), walking k
 //                   upward: the rows D/E/F (AD:2708-3140), the
 //                   THOMASZ_NewType2 forward sweep (MF:4080-4100), then the
@@ -1526,10 +1529,11 @@ __device__ __forceinline__ void cell_rhs_lane(const Dims &d, const StepScalars &
     }
 }
 
-// Explicit kernel of the lane variant: NT / TPL lanes per cell; lane
-// (n, u) = cell cells[n], tracers u*TPL .. u*TPL+TPL-1 of the launch; TI
-// goes to TW, laid out like the tracer state, or with the depth-ordered
-// column walk (S.slot_of) at the cell's level-major slot.
+// Explicit kernel of the lane variant for two or more tracers a launch:
+// NT / TPL lanes per cell; lane (n, u) = cell cells[n], tracers
+// u*TPL .. u*TPL+TPL-1 of the launch; TI goes to TW, laid out like the tracer
+// state, or with the depth-ordered column walk (S.slot_of) at the cell's
+// level-major slot.
 template <bool OPT, int NT, int TPL, bool FAST>
 __global__ void __launch_bounds__(256)
 explicit_lane_kernel(Dims d, StepScalars sc, SharedFields f, TracerSet ts,
@@ -1553,6 +1557,318 @@ explicit_lane_kernel(Dims d, StepScalars sc, SharedFields f, TracerSet ts,
     double TI[TPL];
     cell_rhs_lane<OPT, TPL, FAST>(d, sc, f, tl, x, c.i, c.j, TI, bad);
     store_tpl<TPL>(TW + q * ts.s + t0, TI);
+    if (bad) atomicOr(badflag, 1u);
+}
+
+// ---------------------------------------------------------------------------
+// Explicit kernel of the lane variant for one tracer a launch (every drop-in
+// call): one block per (64 x EY columns, level).  A lane per cell is bound by
+// the FP64 work of the faces (two quotients and a limiter each, every face
+// computed by both its cells) and its stencil loads; here every face is
+// computed once and only where it is needed.  The block finds the tile's
+// solved cells and their computing faces from the masks (ballots, no list in
+// memory), computes the faces into LDS, then gathers the cells.  Both lists
+// are dense, so land and rows below the floor cost a mask byte and no lane.
+// 512 x 512 x 50 sigma, SuperBee: 728 us as a lane per cell, 440 now; 517 x
+// 389 x 37 with 61 % of the cells dry, optimised path: 177 us, 130 now.
+//
+// With two or more tracers the same split loses (2.1 -> 2.9 ms at 1024 x 1024
+// x 40 and 8 tracers): the four stencil loads of a face, 8 TPL bytes a lane at
+// the cell's stride, fill the L1 path, where the lane per cell needs 9 for
+// its four faces.
+constexpr int EX = 64, EY = 8;
+
+// n / R.b through the shared reciprocal, xdiv's steps without its range test:
+// the division's bits unless R is not ok, the quotient overflows (the result
+// is then not finite) or it is non-zero and under 2^-400 (the last bit).  A
+// zero numerator gives +0.
+__device__ __forceinline__ double fdiv(double n, const Recip &R) {
+    const double q0 = n * R.r;
+    return fma(fma(-R.b, q0, n), R.r, q0);
+}
+
+// The U or V face below cell (fi, fj, k), every load before the arithmetic,
+// and what its two cells need of it:
+//   optimised FP64: fl = flux dt, df = the diffusive term's numerator in the
+//     optimised order (AD:5239-5246, 5285-5292);
+//   FAST: fl = the flux, df = conductance times gradient;
+//   otherwise: fl = flux dt, df = the gradient P(high) - P(low).
+template <bool OPT, bool FAST>
+__device__ __forceinline__ void tile_face(const Dims &d, const StepScalars &sc,
+                                          const SharedFields &f, const TracerSet &ts, bool isU,
+                                          int fi, int fj, int k, double &fl, double &df,
+                                          int &bad) {
+    const long c0 = d.idx(fi, fj, k), b = d.idx2(fi, fj);
+    const long st = isU ? d.sj : 1;
+    const double *line = isU ? f.DUX : f.DVY;
+    // the face's high cell is a WorkSize cell, so positions -1 .. +1 are
+    // inside Size; -2 may lie before it, and is then loaded from -1
+    const bool in0 = isU ? fj - 2 >= d.JLB : fi - 2 >= d.ILB;
+    const long far = in0 ? 2 * st : st;
+    const double x0 = ts.P[(c0 - far) * ts.s], p1 = ts.P[(c0 - st) * ts.s],
+                 p2 = ts.P[c0 * ts.s], p3 = ts.P[(c0 + st) * ts.s];
+    const double Q = (isU ? f.Qx : f.Qy)[c0];
+    const uint8_t m0 = f.mask[c0 - far], m1 = f.mask[c0 - st], m2 = f.mask[c0],
+                  m3 = f.mask[c0 + st];
+    const double au = (OPT || FAST) ? (isU ? f.cu : f.cv)[c0] : 0.0;
+    const double du0 = line[b - far], du1 = line[b - st], du2 = line[b], du3 = line[b + st];
+    const double v1 = f.V[c0 - st], v2 = f.V[c0];
+    const bool op0 = in0 && (m0 & M_OPEN), op1 = m1 & M_OPEN, op2 = m2 & M_OPEN,
+               op3 = m3 & M_OPEN;
+    const bool up = Q > 0.0;
+    const bool nearb = up ? !op0 : !op3;
+    const double a = up ? p2 : p1, bb = up ? p1 : p2;   // downstream, upstream
+    double x = 0.0;
+    if (OPT || sc.methodH == UPW1 || (sc.methodH == TVD && sc.tvdH != LIM_PDM)) {
+        // ComputeAdvection1D_TVD_SuperBee_2 (MF:10642-10699) and, on the
+        // non-optimised path, ComputeAdvectionFace's first-order and TVD
+        // branches (MF:10702-10894).  Both flow directions run one path on
+        // selected operands: the reference's D p1 + E p2 is
+        // Q (1 - theta) b + Q theta a in either (a sum of two commutes), and
+        // the first-order flux next to a closed cell has theta = 0.
+        double th = 0.0;
+        if (OPT || sc.methodH == TVD) {
+            const double vup = up ? v1 : v2;
+            const double cr = FAST && OPT ? Q * sc.dt * frcp(vup) : Q * sc.dt / vup;
+            const double s1 = du2 + du1;
+            const double s0 = up ? du1 + du0 : du2 + du3;
+            const double pf = up ? x0 : p3;
+            double rr;
+            if (FAST && OPT) {
+                const double dc = clamp_min_value((a - bb) * frcp(s1));
+                rr = (bb - pf) * frcp(s0) * frcp(dc);
+            } else {
+                const double dc = clamp_min_value((a - bb) / s1);
+                rr = (bb - pf) / s0 / dc;
+            }
+            const double l = OPT ? superbee_theta(rr) : limiter_theta(sc.tvdH, rr, bad);
+            th = nearb ? 0.0 : 0.5 * l * (1.0 - cr);
+        }
+        x = Q * (1.0 - th) * bb + Q * th * a;
+        if (!OPT) {
+            // the reference's zero C and F coefficients
+            const double z = Q * 0.0;
+            x = x + z * (in0 ? x0 : 0.0) + z * p3;
+            if (sc.methodH == TVD && nearb && !sc.up2H) {   // the reference stops here
+                x = 0.0;
+                if (op1 && op2) bad = 1;
+            }
+        }
+    } else if constexpr (!OPT) {
+        const double v0 = f.V[c0 - far], v3 = f.V[c0 + st];
+        const double v[4] = {in0 ? v0 : 1.0, v1, v2, v3};
+        const double du[4] = {in0 ? du0 : 0.0, du1, du2, du3};
+        const bool op[4] = {op0, op1, op2, op3};
+        const double p[4] = {in0 ? x0 : 0.0, p1, p2, p3};
+        const Face4 c = face_general(p, v, du, op, Q, sc.dt, sc.volrelmax, sc.methodH, sc.tvdH,
+                                     sc.up2H, bad);
+        x = c.c * p[0] + c.d * p[1] + c.e * p[2] + c.f * p[3];
+    }
+    if (!(op1 && op2)) x = 0.0;
+    // NoAdvFlux: cleared coefficients (AD:4434-4443)
+    if (!OPT && f.xzero && isU && f.xzero[c0]) x = 0.0;
+    const double g = p2 - p1;
+    fl = FAST ? x : x * sc.dt;
+    df = FAST ? au * g : (OPT ? (isU ? au * g * sc.dt : au * sc.dt * g) : g);
+}
+
+// TI goes to TW, laid out like the tracer state, or with the depth-ordered
+// column walk (S.slot_of) at the cell's level-major slot.  Blocks go round the
+// XCDs by x; XCD q takes the q-th band of G tiles at every level, so that a
+// band's halo rows stay in its L2.
+template <bool OPT, bool FAST>
+__global__ void __launch_bounds__(256)
+explicit_tile_kernel(Dims d, StepScalars sc, SharedFields f, TracerSet ts,
+                     double *__restrict__ TW, SlotColumns S, int tiles_x, int ntiles, int G,
+                     unsigned int *__restrict__ badflag) {
+    constexpr int RPW = EY / 4;                           // rows per wave
+    constexpr int NFU = EX * (EY + 1), NFV = (EX + 1) * EY;
+    constexpr int FSEG = RPW * (EX + EX + 1) + EX;        // a wave's part of the face list
+    constexpr uint32_t UBIT = 0x8000;
+    __shared__ unsigned long long row[EY];                // the tile's solved cells
+    __shared__ int cnt[4], ccnt[4];                       // faces, cells by wave
+    __shared__ uint16_t flist[4][FSEG];                   // UBIT, row, column (7 bits)
+    __shared__ uint16_t clist[4][EX * RPW];
+    __shared__ double2 fx[NFU + NFV];   // U faces [row][column], then V: {fl, df}
+    const int tile = (int)(blockIdx.x & 7) * G + (int)(blockIdx.x >> 3);
+    if (tile >= ntiles) return;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int ty = tile / tiles_x, i0 = d.wILB + (tile - ty * tiles_x) * EX, j0 = d.wJLB + ty * EY;
+    const int k = d.wKLB + (int)blockIdx.y;
+    const long lk = (long)(k - d.KLB) * d.sk, top = (long)(d.wKUB - d.KLB) * d.sk;
+    const bool hz = !sc.vertical1d, fv = hz && !sc.xzflow;
+    uint8_t mk[RPW], mv[RPW], mu = 0;
+    bool solved[RPW];
+#pragma unroll
+    for (int q = 0; q < RPW; ++q) {
+        const int r = wave * RPW + q, i = i0 + lane, j = j0 + r;
+        const bool in = i <= d.wIUB && j <= d.wJUB;
+        mk[q] = mv[q] = 0;
+        solved[q] = false;
+        if (in) {
+            const long b = d.idx2(i, j);
+            mk[q] = f.mask[b + lk];
+            if (lane == EX - 1) mv[q] = f.mask[b + lk + 1];
+            if (r == EY - 1) mu = f.mask[b + lk + d.sj];
+            // a row the reference solves: MF:4086, and not an inert land row
+            const uint8_t mt = f.mask[b + top];
+            const int ks = f.kstart[b];
+            solved[q] = (mt & M_WATER) && k >= ks;
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < RPW; ++q) {
+        const unsigned long long w = __ballot(solved[q]);
+        if (lane == 0) row[wave * RPW + q] = w;
+    }
+    __syncthreads();
+    unsigned long long any = 0;
+#pragma unroll
+    for (int r = 0; r < EY; ++r) any |= row[r];
+    if (!any) return;
+    {
+        const unsigned long long below = (1ull << lane) - 1ull;
+        int nf = 0, nc = 0;       // the wave's so far
+        unsigned long long wm = wave > 0 ? row[wave * RPW - 1] : 0ull;
+#pragma unroll
+        for (int q = 0; q < RPW; ++q) {
+            const int r = wave * RPW + q;
+            const unsigned long long w = __ballot(solved[q]);
+            // the faces of the tile's solved cells: U (row r, and the one
+            // above the last row), V (and the one past the last column)
+            const bool u = hz && (mk[q] & M_CFU) && (((w | wm) >> lane) & 1);
+            const bool v = fv && (mk[q] & M_CFV) && (((w | (w << 1)) >> lane) & 1);
+            const bool vh = fv && lane == EX - 1 && (mv[q] & M_CFV) && (w >> 63);
+            const unsigned long long bu = __ballot(u), bv = __ballot(v), bw = __ballot(vh);
+            const uint32_t id = (uint32_t)(r << 7) | (uint32_t)lane;
+            if (u) flist[wave][nf + __popcll(bu & below)] = (uint16_t)(UBIT | id);
+            nf += __popcll(bu);
+            if (v) flist[wave][nf + __popcll(bv & below)] = (uint16_t)id;
+            nf += __popcll(bv);
+            if (vh) flist[wave][nf] = (uint16_t)(id + 1);
+            nf += bw ? 1 : 0;
+            if (solved[q]) clist[wave][nc + __popcll(w & below)] = (uint16_t)id;
+            nc += __popcll(w);
+            if (r == EY - 1) {
+                const bool uh = hz && (mu & M_CFU) && solved[q];
+                const unsigned long long bh = __ballot(uh);
+                if (uh) flist[wave][nf + __popcll(bh & below)] = (uint16_t)(UBIT | (id + 128u));
+                nf += __popcll(bh);
+            }
+            wm = w;
+        }
+        if (lane == 0) {
+            cnt[wave] = nf;
+            ccnt[wave] = nc;
+        }
+    }
+    __syncthreads();
+    // entry n of the four waves' lists
+    const int f1 = cnt[0], f2 = f1 + cnt[1], f3 = f2 + cnt[2], f4 = f3 + cnt[3];
+    const int c1 = ccnt[0], c2 = c1 + ccnt[1], c3 = c2 + ccnt[2], c4 = c3 + ccnt[3];
+    auto where = [](int n, int n1, int n2, int n3, int seg) {
+        return n < n1 ? n : (n < n2 ? seg + n - n1 : (n < n3 ? 2 * seg + n - n2
+                                                              : 3 * seg + n - n3));
+    };
+    // a cell's loads; a lane's first cell is loaded ahead of the faces
+    struct Cell {
+        uint32_t id;
+        uint8_t mc, mu1, mv1;
+        double p, v, vold;
+    };
+    auto load_cell = [&](int n) {
+        Cell c;
+        c.id = (&clist[0][0])[where(n, c1, c2, c3, EX * RPW)];
+        const long x = d.idx2(i0 + (int)(c.id & 127), j0 + (int)(c.id >> 7)) + lk;
+        c.p = ts.P[x * ts.s];
+        c.mc = f.mask[x];
+        c.mu1 = f.mask[x + d.sj];
+        c.mv1 = f.mask[x + 1];
+        c.v = f.V[x];
+        c.vold = f.Vold[x];
+        return c;
+    };
+    Cell cell{};
+    if ((int)threadIdx.x < c4) cell = load_cell(threadIdx.x);
+    int bad = 0;
+    for (int q = threadIdx.x; q < f4; q += 256) {
+        const uint32_t id = (&flist[0][0])[where(q, f1, f2, f3, FSEG)];
+        const bool isU = id & UBIT;
+        const int r = (id >> 7) & 0xff, c = id & 127;
+        double fl, df;
+        tile_face<OPT, FAST>(d, sc, f, ts, isU, i0 + c, j0 + r, k, fl, df, bad);
+        fx[isU ? r * EX + c : NFU + r * (EX + 1) + c] = make_double2(fl, df);
+    }
+    __syncthreads();
+    const double dt = sc.dt;
+    for (int q = threadIdx.x; q < c4; q += 256) {
+        if (q >= 256) cell = load_cell(q);
+        const int r = cell.id >> 7, c = cell.id & 127;
+        const long b2 = d.idx2(i0 + c, j0 + r), x = b2 + lk;
+        const long xt = S.slot_of ? (long)(k - d.KLB) * S.ncols + S.slot_of[b2] : x;
+        const double2 *uo = fx + r * EX + c, *vo = fx + NFU + r * (EX + 1) + c;
+        const double pk = cell.p, vk = cell.v;
+        const bool open = cell.mc & M_OPEN;
+        const bool cfu0 = hz && (cell.mc & M_CFU), cfu1 = hz && (cell.mu1 & M_CFU);
+        const bool cfv0 = fv && (cell.mc & M_CFV), cfv1 = fv && (cell.mv1 & M_CFV);
+        const double2 z = make_double2(0.0, 0.0);
+        const double2 u0 = cfu0 ? uo[0] : z, u1 = cfu1 ? uo[EX] : z;
+        const double2 w0 = cfv0 ? vo[0] : z, w1 = cfv1 ? vo[1] : z;
+        if constexpr (FAST) {
+            const double ivk = frcp(vk), dtv = dt * ivk;
+            double TI = open ? pk * (cell.vold * ivk) : pk;
+            disch_ti(f, x, open, pk, dt, vk, TI);
+            TI = TI - u0.y * dtv + u1.y * dtv - w0.y * dtv + w1.y * dtv;
+            const bool nud = !OPT && f.nadv;
+            double A = nud ? 0.0 : TI;
+            A = A + u0.x * dtv - u1.x * dtv + w0.x * dtv - w1.x * dtv;
+            if (nud) f.nadv[x * ts.s] = A;
+            TW[xt * ts.s] = nud ? TI : A;
+        } else {
+            // every quotient by V shares its reciprocal
+            const Recip Rv = recip(vk);
+            double TI0 = open ? pk * xdiv(cell.vold, Rv) : pk;
+            disch_ti(f, x, open, pk, dt, vk, TI0);
+            // the non-optimised path weights the gradients with au dt/V
+            // (AD:5178-5197, 5335-5350)
+            double wu0 = 0.0, wu1 = 0.0, wv0 = 0.0, wv1 = 0.0;
+            if constexpr (!OPT) {
+                const double au0 = f.cu[x], au1 = f.cu[x + d.sj];
+                const double av0 = f.cv[x], av1 = f.cv[x + 1];
+                wu0 = cfu0 ? au0 * dt : 0.0;
+                wu1 = cfu1 ? au1 * dt : 0.0;
+                wv0 = cfv0 ? av0 * dt : 0.0;
+                wv1 = cfv1 ? av1 * dt : 0.0;
+            }
+            // with nudging the advective terms gather in AdvectionTi, from
+            // zero (AD:4154-4157, 4665-4668, 5043-5046)
+            const bool nud = !OPT && f.nadv;
+            double TI, A;
+            // the terms in the order the reference's loops deliver them; a
+            // face that does not compute adds a zero
+            auto terms = [&](auto quot) {
+                TI = TI0;
+                TI = TI - (OPT ? quot(u0.y, cfu0) : quot(wu0, cfu0) * u0.y);
+                TI = TI + (OPT ? quot(u1.y, cfu1) : quot(wu1, cfu1) * u1.y);
+                TI = TI - (OPT ? quot(w0.y, cfv0) : quot(wv0, cfv0) * w0.y);
+                TI = TI + (OPT ? quot(w1.y, cfv1) : quot(wv1, cfv1) * w1.y);
+                A = nud ? 0.0 : TI;
+                A = A + quot(u0.x, cfu0);
+                A = A - quot(u1.x, cfu1);
+                A = A + quot(w0.x, cfv0);
+                A = A - quot(w1.x, cfv1);
+            };
+            terms([&](double n, bool) { return fdiv(n, Rv); });
+            // fdiv's bits are the division's for every term a sum of this
+            // size can show: one test of the sums instead of one per term
+            const double m = fabs(nud ? TI + A : A);
+            if (!(Rv.ok & (m < 0x1p1000) & ((m >= 0x1p-300) | (m == 0.0))))
+                terms([&](double n, bool on) { return on ? n / vk : 0.0; });
+            if (nud) f.nadv[x * ts.s] = A;
+            TW[xt * ts.s] = nud ? TI : A;
+        }
+    }
     if (bad) atomicOr(badflag, 1u);
 }
 
@@ -2534,6 +2850,20 @@ slot_map_kernel(const uint32_t *__restrict__ cols, long nc, int32_t *__restrict_
 
 // Lane-variant launches with TPL tracers per lane (1, 2, 4 or 8 dividing NT;
 // 0 picks the default: 4 in the explicit kernel, 2 in the column walk).
+// One tracer: tiles, with every face computed once.
+template <bool OPT, bool FAST>
+static int launch_explicit_tiles(const Dims &d, const StepScalars &sc, const SharedFields &f,
+                                 const TracerSet &ts, const SolveLists &l, double *TW,
+                                 unsigned int *bad, hipStream_t s) {
+    const int ni = d.wIUB - d.wILB + 1, nj = d.wJUB - d.wJLB + 1, nk = d.wKUB - d.wKLB + 1;
+    const int tiles_x = (ni + EX - 1) / EX, ntiles = tiles_x * ((nj + EY - 1) / EY);
+    const int G = (ntiles + 7) / 8;
+    hipLaunchKernelGGL((explicit_tile_kernel<OPT, FAST>), dim3(8 * G, nk), dim3(256), 0, s, d,
+                       sc, f, ts, TW, l.slot, tiles_x, ntiles, G, bad);
+    HIPCHK(hipGetLastError());
+    return MGPU_SUCCESS;
+}
+
 template <bool OPT, int NT, int TPL, bool FAST>
 static int launch_explicit_tpl(const Dims &d, const StepScalars &sc, const SharedFields &f,
                                const TracerSet &ts, const SolveLists &l, double *TW,
@@ -2627,6 +2957,9 @@ template <bool OPT, int NT, bool FAST>
 static int launch_explicit_lanes(int want, const Dims &d, const StepScalars &sc,
                                  const SharedFields &f, const TracerSet &ts, const SolveLists &l,
                                  double *TW, unsigned int *bad, hipStream_t s) {
+    if constexpr (NT == 1) return launch_explicit_tiles<OPT, FAST>(d, sc, f, ts, l, TW, bad, s);
+    else {
+    if (!l.cells) return MGPU_ERR_STATE;
     switch (lane_tpl<NT>(want, 4)) {
         case 8: if constexpr (NT % 8 == 0) return launch_explicit_tpl<OPT, NT, 8, FAST>(d, sc, f, ts, l, TW, bad, s); break;
         case 4: if constexpr (NT % 4 == 0) return launch_explicit_tpl<OPT, NT, 4, FAST>(d, sc, f, ts, l, TW, bad, s); break;
@@ -2634,6 +2967,7 @@ static int launch_explicit_lanes(int want, const Dims &d, const StepScalars &sc,
         default: break;
     }
     return launch_explicit_tpl<OPT, NT, 1, FAST>(d, sc, f, ts, l, TW, bad, s);
+    }
 }
 
 template <bool OPT, int NT, bool FAST>

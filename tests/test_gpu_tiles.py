@@ -1,0 +1,69 @@
+"""The one-tracer explicit kernel at the edges of its 64 x 8 tiles (GPU), equal
+to the oracle on every cell: extents around a tile, one level, every branch of
+the face, fields with exact zeros and with values far below 1."""
+import numpy as np
+import pytest
+
+from mohid_amd import constants as C
+from mohid_amd import fixtures as fx
+from oracle import oracle as ora
+
+from .cases import GRID
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(case, props, optimize):
+    from mohid_amd.advection_diffusion import AdvectionDiffusion
+    case.params["Optimize"] = optimize
+    inst = ora.Instance(case, nthreads=1)
+    gpu = AdvectionDiffusion(case.size, case.worksize, case.geom)
+    got = [np.array(p, order="F", copy=True) for p in props]
+    ref = [np.array(p, order="F", copy=True) for p in props]
+    for s in range(2):
+        for t in range(len(props)):
+            assert inst.step(ref[t], first_property=t == 0,
+                             now=(s + 1) * case.params["DTProp"]) == 0
+            gpu(got[t], case.hydro, case.params, first_property=t == 0)
+            assert np.array_equal(got[t], ref[t]), (s, t)
+    gpu.kill()
+    inst.close()
+
+
+@pytest.mark.parametrize("optimize", (False, True))
+@pytest.mark.parametrize("ni,nj,nk,kfloor,land", [
+    (3, 3, 1, (1, 1), 0.0), (63, 7, 3, (1, 3), 0.2), (64, 8, 2, (1, 1), 0.0),
+    (65, 9, 4, (2, 4), 0.4), (129, 17, 5, (1, 5), 0.3), (2, 40, 6, (1, 6), 0.1)])
+def test_extents(ni, nj, nk, kfloor, land, optimize):
+    case = fx.make_case(fx.config("c3", ni=ni, nj=nj, nk=nk, kfloor=kfloor, land_frac=land,
+                                  tracers=("temperature", "lognormal"), **GRID))
+    _check(case, case.tracers, optimize)
+
+
+@pytest.mark.parametrize("method,limiter,up2", [
+    (C.UPWIND_ORDER1, C.SUPERBEE, False), (C.P2_TVD, C.MINMOD, True),
+    (C.P2_TVD, C.VANLEER, True), (C.P2_TVD, C.MUSCL, True), (C.P2_TVD, C.SUPERBEE, True),
+    (C.P2_TVD, C.PDM, True), (C.CENTRAL_DIF, C.SUPERBEE, False)])
+def test_faces(method, limiter, up2):
+    case = fx.make_case(fx.config("c3", ni=70, nj=19, nk=5, kfloor=(1, 5), land_frac=0.3,
+                                  tracers=("lognormal",), **GRID))
+    case.params.update(AdvMethodH=method, TVDLimitationH=limiter, Upwind2H=up2)
+    _check(case, case.tracers, False)
+
+
+@pytest.mark.parametrize("optimize", (False, True))
+def test_zero_and_small_values(optimize):
+    """Exact zeros beside a patch, and the patch at 1e-200: every quotient is
+    zero, or too small for the shared-reciprocal form."""
+    case = fx.make_case(fx.config("c3", ni=70, nj=19, nk=5, kfloor=(1, 5), land_frac=0.3,
+                                  tracers=("lognormal", "lognormal"), **GRID))
+    wet = case.hydro["WaterPoints3D"] == 1
+    props = []
+    for scale in (1.0, 1e-200):
+        p = np.array(case.tracers[0], order="F", copy=True)
+        far = np.zeros_like(wet)
+        far[30:] = True
+        p[wet & far] = 0.0
+        p[wet & ~far] *= scale
+        props.append(p)
+    _check(case, props, optimize)

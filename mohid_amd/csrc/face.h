@@ -65,6 +65,15 @@ __device__ __forceinline__ double xdiv(double a, const Recip &R) {
     return a / R.b;
 }
 
+// n / R.b through the shared reciprocal, xdiv's steps without its range test:
+// the division's bits unless R is not ok, the quotient overflows (the result
+// is then not finite) or it is non-zero and under 2^-400 (the last bit).  A
+// zero numerator gives +0.
+__device__ __forceinline__ double fdiv(double n, const Recip &R) {
+    const double q0 = n * R.r;
+    return fma(fma(-R.b, q0, n), R.r, q0);
+}
+
 __device__ __forceinline__ double dmin(double a, double b) { return a < b ? a : b; }
 __device__ __forceinline__ double dmax(double a, double b) { return a > b ? a : b; }
 

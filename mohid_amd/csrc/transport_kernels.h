@@ -38,6 +38,8 @@
 // in the reference.
 #pragma once
 
+#include <type_traits>
+
 #include "face.h"
 #include "mgpu_internal.h"
 
@@ -151,6 +153,11 @@ __device__ __forceinline__ void face_pos(int f, int &fi, int &fj, bool &isU, int
 __device__ __forceinline__ long xcd_tile(long b, long n) {
     const long q = n / 8, r = n % 8, x = b % 8, idx = b / 8;
     return x * q + (x < r ? x : r) + idx;
+}
+
+__device__ __forceinline__ long xcd_tile32(unsigned b, unsigned n) {
+    const unsigned q = n >> 3, r = n & 7, x = b & 7;
+    return (long)(x * q + (x < r ? x : r) + (b >> 3));
 }
 
 // For a grid over (level, tile) pairs: XCD x takes a contiguous segment of
@@ -863,10 +870,127 @@ struct RowSet {
     double D[NT], E[NT], F[NT], TI[NT];
 };
 
+// What the row of cell (k) shares between tracers: dt/V, VolumeVariation's
+// diagonal, the two W faces' weighted conductances, flags.
+struct RowShared {
+    double vk, dtk, E0, a1, a2;
+    bool cfwB, cfwT, land, vdif, open;
+};
+
+// qz1: Qz of the face above; cwB, cwT: conductances of the faces below and
+// above, mT the mask above (read only where the mask says so).
+template <bool FAST, typename CW>
+__device__ __forceinline__ RowShared row_shared(const StepScalars &sc, const SharedFields &f,
+                                                long x, int k, int KUB, double vk, uint8_t mk,
+                                                uint8_t mT, double qz1, CW cw) {
+    const double dt = sc.dt;
+    RowShared r;
+    r.vk = vk;
+    r.dtk = FAST ? dt * frcp(vk) : dt / vk;
+    r.open = mk & M_OPEN;
+    r.E0 = 1.0;
+    if (k == KUB && r.open && !sc.hreset) r.E0 = 1.0 + r.dtk * qz1;
+    if (!sc.hreset) disch_e(f, x, r.open, dt, vk, r.E0);   // AD:4100-4102
+    r.cfwB = sc.vert && (mk & M_CFW);
+    r.cfwT = sc.vert && k < KUB && (mT & M_CFW);
+    r.a2 = r.cfwB ? (FAST ? cw(0) * r.dtk : cw(0) * dt / vk) : 0.0;
+    r.a1 = r.cfwT ? (FAST ? cw(1) * r.dtk : cw(1) * dt / vk) : 0.0;
+    r.land = mk & M_LAND;
+    r.vdif = !(mk & M_SDV);   // SmallDepthCell (AD:2733, 2813-2907)
+    return r;
+}
+
+// One tracer's row of cell x (level k of the column at base): D/E/F, and TI
+// completed with the vertical terms.  ts at the tracer; p: its values at
+// levels k-1 .. k+2; fb, ft: the coefficients of the faces below and above.
+// ONE: a launch of one tracer (nudging).  With OBC the open cells of boundary
+// columns take the open boundary rows.
+template <bool OPT, bool FAST, bool OBC, bool ONE>
+__device__ __forceinline__ void row_terms(const Dims &d, const StepScalars &sc,
+                                          const SharedFields &f, const TracerSet &ts, long base,
+                                          long x, int k, const RowShared &r, const double p[4],
+                                          const VCoef &fb, const VCoef &ft, double &D, double &E,
+                                          double &F, double &TI, int &bad) {
+    const double dt = sc.dt, dtk = r.dtk, vk = r.vk;
+    const bool cfwB = r.cfwB, cfwT = r.cfwT;
+    const double pm = p[0], pk = p[1], pp = p[2];
+    E = r.E0;
+    D = 0.0;
+    F = 0.0;
+    if (cfwB && r.vdif) {
+        if (OPT) {
+            if (sc.thV > 0.0) { D = D - r.a2; E = E + r.a2; }
+            else TI = TI - r.a2 * (pk - pm);
+        } else {
+            D = D - r.a2 * sc.thV;
+            E = E + r.a2 * sc.thV;
+            TI = TI - r.a2 * (pk - pm) * (1.0 - sc.thV);
+        }
+    }
+    if (cfwT && r.vdif) {
+        if (OPT) {
+            if (sc.thV > 0.0) { E = E + r.a1; F = F - r.a1; }
+            else TI = TI + r.a1 * (pp - pk);
+        } else {
+            E = E + r.a1 * sc.thV;
+            F = F - r.a1 * sc.thV;
+            TI = TI + r.a1 * (pp - pk) * (1.0 - sc.thV);
+        }
+    }
+    // nudging: the advective terms in AdvectionTi/D/E/F (VerticalAdvection_Nudge,
+    // AD:3211-3350), joined to the rows with the column's weight on open
+    // points (AdvectionNudging, AD:2055-2062); the explicit kernel left
+    // the horizontal ones in nadv
+    const bool nud = !OPT && ONE && f.nadv != nullptr;
+    double aT = nud ? f.nadv[x * ts.s] : 0.0, aD = 0.0, aE = 0.0, aF = 0.0;
+    if (sc.vert && !sc.vertical1d) {
+        if (sc.impAdvV && nud) {
+            if (cfwB) { aD = aD - fb.d * dtk; aE = aE - fb.e * dtk; }
+            if (cfwT) { aE = aE + ft.d * dtk; aF = aF + ft.e * dtk; }
+        } else if (sc.impAdvV) {
+            if (cfwB) { D = D - fb.d * dtk; E = E - fb.e * dtk; }
+            if (cfwT) { E = E + ft.d * dtk; F = F + ft.e * dtk; }
+        } else if (OPT) {
+            if (FAST) {
+                if (cfwB) TI = TI + (fb.d * pm + fb.e * pk) * dtk;
+                if (cfwT) TI = TI - (ft.d * pk + ft.e * pp) * dtk;
+            } else {
+                if (cfwB) TI = TI + (fb.d * pm + fb.e * pk) * dt / vk;
+                if (cfwT) TI = TI - (ft.d * pk + ft.e * pp) * dt / vk;
+            }
+        } else {
+            if (cfwB) {
+                const double pmm = (fb.c == 0.0 || k - 2 < d.KLB) ? 0.0 : ts.P[(x - 2 * d.sk) * ts.s];
+                const double fl = fb.c * pmm + fb.d * pm + fb.e * pk + fb.f * pp;
+                if (nud) aT = aT + fl * dt / vk;
+                else TI = TI + fl * dt / vk;
+            }
+            if (cfwT) {
+                const double fl = ft.c * pm + ft.d * pk + ft.e * pp + ft.f * p[3];
+                if (nud) aT = aT - fl * dt / vk;
+                else TI = TI - fl * dt / vk;
+            }
+        }
+    }
+    if (nud && r.open) {
+        const double n = f.nw[base];
+        TI = TI + n * aT;
+        D = D + n * aD;
+        E = E + n * aE;
+        F = F + n * aF;
+    }
+    if constexpr (OBC) {
+        // boundary column (base is its (i, j) index: KLB is 0), levels
+        // |KFloorZ|..KUB (AD:5437-5444)
+        if (f.obc.bp[base] == 1 && r.open && k >= abs(f.obc.kfloor[base]))
+            obc_row(d, sc, f, ts.P, ts.s, x, base, vk, TI, D, E, F, bad);
+    }
+    if (r.land) TI = MGPU_NULL_REAL;
+}
+
 // Row k of the column: assembles D/E/F and completes TI with the vertical
 // terms, then one forward-sweep step of THOMASZ_NewType2; slides the
-// windows up one level.  With OBC the open cells of boundary columns take
-// the open boundary rows.  With `rows` the finished rows go there and no
+// windows up one level.  With `rows` the finished rows go there and no
 // sweep step is taken (Wo, Go, the carried W and G are left alone).
 template <bool OPT, int NT, bool FAST, bool OBC = false>
 __device__ __forceinline__ void column_row(const Dims &d, const StepScalars &sc,
@@ -878,107 +1002,25 @@ __device__ __forceinline__ void column_row(const Dims &d, const StepScalars &sc,
                                            int &bad, RowSet<NT> *rows = nullptr) {
     const long sk = d.sk;
     const int KUB = d.wKUB;
-    const double dt = sc.dt;
     auto inK = [&](int kk) { return kk >= d.KLB && kk <= d.KUB; };
     const long x = base + k * sk;
-    const double vk = c.wv[1];
-    const uint8_t mk = c.wm[1];
     // coefficients of the face above (k, k+1): stencil k-1 .. k+2
     VCoef ft[NT];
+    const double qz1 = inK(k + 1) ? f.Qz[x + sk] : 0.0;
     {
         const bool o4[4] = {(c.wm[0] & M_OPEN) != 0, (c.wm[1] & M_OPEN) != 0,
                             (c.wm[2] & M_OPEN) != 0, (c.wm[3] & M_OPEN) != 0};
-        vface_coefs<OPT, NT, FAST>(sc, c.wp, c.wv, c.wdu, o4, inK(k + 1) ? f.Qz[x + sk] : 0.0,
-                                   vflux && k < KUB, ft, bad);
+        vface_coefs<OPT, NT, FAST>(sc, c.wp, c.wv, c.wdu, o4, qz1, vflux && k < KUB, ft, bad);
     }
-    // row values shared by all tracers
-    const double dtk = FAST ? dt * frcp(vk) : dt / vk;
-    double E0 = 1.0;
-    if (k == KUB && (mk & M_OPEN) && !sc.hreset) E0 = 1.0 + dtk * f.Qz[x + sk];
-    if (!sc.hreset) disch_e(f, x, mk & M_OPEN, dt, vk, E0);   // AD:4100-4102
-    const bool cfwB = sc.vert && (mk & M_CFW);
-    const bool cfwT = sc.vert && k < KUB && (c.wm[2] & M_CFW);
-    const double a2 = cfwB ? (FAST ? f.cw[x] * dtk : f.cw[x] * dt / vk) : 0.0;
-    const double a1 = cfwT ? (FAST ? f.cw[x + sk] * dtk : f.cw[x + sk] * dt / vk) : 0.0;
-    const bool land = mk & M_LAND;
-    const bool vdif = !(mk & M_SDV);   // SmallDepthCell (AD:2733, 2813-2907)
+    const RowShared r =
+        row_shared<FAST>(sc, f, x, k, KUB, c.wv[1], c.wm[1], c.wm[2], qz1,
+                         [&](int up) { return f.cw[up ? x + sk : x]; });
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-        const double pk = c.wp[t][1], pm = c.wp[t][0], pp = c.wp[t][2];
-        double TI = TIk[t];
-        double E = E0, D = 0.0, F = 0.0;
-        if (cfwB && vdif) {
-            if (OPT) {
-                if (sc.thV > 0.0) { D = D - a2; E = E + a2; }
-                else TI = TI - a2 * (pk - pm);
-            } else {
-                D = D - a2 * sc.thV;
-                E = E + a2 * sc.thV;
-                TI = TI - a2 * (pk - pm) * (1.0 - sc.thV);
-            }
-        }
-        if (cfwT && vdif) {
-            if (OPT) {
-                if (sc.thV > 0.0) { E = E + a1; F = F - a1; }
-                else TI = TI + a1 * (pp - pk);
-            } else {
-                E = E + a1 * sc.thV;
-                F = F - a1 * sc.thV;
-                TI = TI + a1 * (pp - pk) * (1.0 - sc.thV);
-            }
-        }
-        // nudging: the advective terms in AdvectionTi/D/E/F (VerticalAdvection_Nudge,
-        // AD:3211-3350), joined to the rows with the column's weight on open
-        // points (AdvectionNudging, AD:2055-2062); the explicit kernel left
-        // the horizontal ones in nadv
-        const bool nud = !OPT && NT == 1 && f.nadv != nullptr;
-        double aT = nud ? f.nadv[x * ts.s + t] : 0.0, aD = 0.0, aE = 0.0, aF = 0.0;
-        if (sc.vert && !sc.vertical1d) {
-            if (sc.impAdvV && nud) {
-                if (cfwB) { aD = aD - c.fb[t].d * dtk; aE = aE - c.fb[t].e * dtk; }
-                if (cfwT) { aE = aE + ft[t].d * dtk; aF = aF + ft[t].e * dtk; }
-            } else if (sc.impAdvV) {
-                if (cfwB) { D = D - c.fb[t].d * dtk; E = E - c.fb[t].e * dtk; }
-                if (cfwT) { E = E + ft[t].d * dtk; F = F + ft[t].e * dtk; }
-            } else if (OPT) {
-                if (FAST) {
-                    if (cfwB) TI = TI + (c.fb[t].d * pm + c.fb[t].e * pk) * dtk;
-                    if (cfwT) TI = TI - (ft[t].d * pk + ft[t].e * pp) * dtk;
-                } else {
-                    if (cfwB) TI = TI + (c.fb[t].d * pm + c.fb[t].e * pk) * dt / vk;
-                    if (cfwT) TI = TI - (ft[t].d * pk + ft[t].e * pp) * dt / vk;
-                }
-            } else {
-                if (cfwB) {
-                    const double pmm =
-                        (c.fb[t].c == 0.0 || k - 2 < d.KLB) ? 0.0 : ts.P[(x - 2 * sk) * ts.s + t];
-                    const double fl =
-                        c.fb[t].c * pmm + c.fb[t].d * pm + c.fb[t].e * pk + c.fb[t].f * pp;
-                    if (nud) aT = aT + fl * dt / vk;
-                    else TI = TI + fl * dt / vk;
-                }
-                if (cfwT) {
-                    const double fl = ft[t].c * pm + ft[t].d * pk + ft[t].e * pp +
-                                      ft[t].f * c.wp[t][3];
-                    if (nud) aT = aT - fl * dt / vk;
-                    else TI = TI - fl * dt / vk;
-                }
-            }
-        }
-        if (nud && (mk & M_OPEN)) {
-            const double n = f.nw[base];
-            TI = TI + n * aT;
-            D = D + n * aD;
-            E = E + n * aE;
-            F = F + n * aF;
-        }
-        if constexpr (OBC) {
-            // boundary column (base is its (i, j) index: KLB is 0), levels
-            // |KFloorZ|..KUB (AD:5437-5444)
-            if (f.obc.bp[base] == 1 && (mk & M_OPEN) && k >= abs(f.obc.kfloor[base]))
-                obc_row(d, sc, f, ts.P + t, ts.s, x, base, vk, TI, D, E, F, bad);
-        }
-        if (land) TI = MGPU_NULL_REAL;
+        double D, E, F, TI = TIk[t];
+        const TracerSet t1{ts.P + t, nullptr, ts.s, nullptr};
+        row_terms<OPT, FAST, OBC, NT == 1>(d, sc, f, t1, base, x, k, r, c.wp[t], c.fb[t], ft[t],
+                                           D, E, F, TI, bad);
         if (rows) {
             rows->D[t] = D; rows->E[t] = E; rows->F[t] = F; rows->TI[t] = TI;
             c.fb[t] = ft[t];
@@ -1577,15 +1619,6 @@ explicit_lane_kernel(Dims d, StepScalars sc, SharedFields f, TracerSet ts,
 // the cell's stride, fill the L1 path, where the lane per cell needs 9 for
 // its four faces.
 constexpr int EX = 64, EY = 8;
-
-// n / R.b through the shared reciprocal, xdiv's steps without its range test:
-// the division's bits unless R is not ok, the quotient overflows (the result
-// is then not finite) or it is non-zero and under 2^-400 (the last bit).  A
-// zero numerator gives +0.
-__device__ __forceinline__ double fdiv(double n, const Recip &R) {
-    const double q0 = n * R.r;
-    return fma(fma(-R.b, q0, n), R.r, q0);
-}
 
 // The U or V face below cell (fi, fj, k), every load before the arithmetic,
 // and what its two cells need of it:
@@ -2249,6 +2282,222 @@ column_pipe_kernel(Dims d, StepScalars sc, SharedFields f, TracerSet ts,
 }
 
 // ---------------------------------------------------------------------------
+// Column walk for few columns (quad_columns).  A lane per (column, tracer)
+// leaves the chip short of waves, and each lane then waits on its own serial chain: the row
+// assembly (some 200 FP64 instructions a level) is far longer than the
+// recurrence itself.  Here the four lanes of a quad share a column: each
+// assembles the row of one of four consecutive levels, then the sweep runs
+// through the quad, one level a step, W and G handed on by DPP; the back
+// substitution the same way down.  W and G stay in LDS (a pair per lane and
+// group of four levels), so the walk has no scratch traffic.  The operations
+// of a row are those of column_row; a row below the column's first one is the
+// identity with TI = 0, which leaves the carried W and G at zero.
+template <int CTRL>
+__device__ __forceinline__ double quad_perm(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
+constexpr int QUAD_UP = 0 | (0 << 2) | (1 << 4) | (2 << 6);   // from the lane below
+template <int S>
+__device__ __forceinline__ double quad_lane(double v) {
+    return quad_perm<S * 0x55>(v);
+}
+
+// One lane's inputs of level k (clamped into Size; levels outside hold what
+// column_begin gives them).
+struct QuadIn {
+    double TI, p[4], v[4], du[4], qz1, cwB, cwT;
+    uint8_t m[4];
+};
+
+template <bool SLOT>
+__device__ __forceinline__ void quad_load(const Dims &d, const StepScalars &sc,
+                                          const SharedFields &f, const TracerSet &ts,
+                                          const double *tw, const SlotColumns &S, long base,
+                                          long n, int k, double dux, double dvy, QuadIn &q) {
+    const int kc = k < d.KLB ? d.KLB : k;
+    const long x = base + kc * d.sk, xs = (long)(kc - d.KLB) * S.ncols + n;
+    const double *V = SLOT ? S.V : f.V, *DWZ = SLOT ? S.DWZ : f.DWZ;
+    const uint8_t *mask = SLOT ? S.mask : f.mask;
+    q.TI = sc.hreset ? ts.P[x * ts.s] : tw[(SLOT ? xs : x) * ts.s];
+#pragma unroll
+    for (int o = 0; o < 4; ++o) {
+        const int kk = kc - 1 + o;
+        const bool in = kk >= d.KLB && kk <= d.KUB;
+        const int kl = in ? kk : kc;
+        const long y = base + kl * d.sk, ys = SLOT ? (long)(kl - d.KLB) * S.ncols + n : y;
+        const double p = ts.P[y * ts.s], v = V[ys], du = DWZ[ys];
+        const uint8_t m = mask[ys];
+        q.p[o] = in ? p : 0.0;
+        q.v[o] = in ? v : 1.0;
+        q.du[o] = in ? du : 0.0;
+        q.m[o] = in ? m : (uint8_t)0;
+    }
+    // k <= WorkSize KUB, so the level above is inside Size
+    if (SLOT) {
+        q.qz1 = S.Qz[xs];
+        q.cwT = (S.sV * S.Kz[xs] + S.bV) * dux * dvy / S.DZZ[xs];
+        q.cwB = 0.0;
+    } else {
+        q.qz1 = f.Qz[x + d.sk];
+        q.cwB = f.cw[x];
+        q.cwT = f.cw[x + d.sk];
+    }
+}
+
+template <bool OPT, int NT, bool FAST, bool OBC, bool SLOT>
+__global__ void __launch_bounds__(64)
+column_quad_kernel(Dims d, StepScalars sc, SharedFields f, TracerSet ts,
+                   const uint32_t *__restrict__ cols, long ncols, const double *__restrict__ TW,
+                   SlotColumns S, unsigned long long *__restrict__ zero_pivots,
+                   unsigned int *__restrict__ badflag) {
+    extern __shared__ double2 wg[];       // [group][lane]
+    const int lane = threadIdx.x, l = lane & 3;
+    const long blk = SLOT ? (long)blockIdx.x : xcd_tile32(blockIdx.x, gridDim.x);
+    const long g = blk * 16 + (lane >> 2);
+    const long nn = g / NT;
+    const bool act = nn < ncols;
+    // lanes past the end walk the last column and store nothing: the quads of
+    // a wave stay together
+    const long n = act ? nn : ncols - 1;
+    const int t = (int)(g - nn * NT);
+    const int KUB = d.wKUB;
+    const long base = cols[n], sk = d.sk, s = ts.s;
+    const int ks = SLOT ? S.ks[n] : f.kstart[base];
+    const TracerSet t1{ts.P + t, ts.out + t, s, ts.G0 ? ts.G0 + t : nullptr};
+    const double *tw = TW + t;
+    int bad = 0;
+    const bool columnBuild =   // AD:2982/3004
+        (SLOT ? S.mask[(long)(KUB - d.KLB) * S.ncols + n] : f.mask[base + KUB * sk]) & M_OPEN;
+    const bool vflux = sc.vert && !sc.vertical1d && columnBuild;
+    const double dux = SLOT ? S.dux[n] : 0.0, dvy = SLOT ? S.dvy[n] : 0.0;
+    // the groups end at KUB and begin one level below the wave's lowest first
+    // row, whose upper face the row above needs
+    const int ng = (KUB - (wave_min(ks) - 1)) / 4 + 1;
+    const int k0 = KUB - 4 * ng + 1 + l;
+    double W = 0.0, G = 0.0;              // carried, the same in the quad
+    VCoef fc{0.0, 0.0, 0.0, 0.0};         // the face below the group
+    double cwc = 0.0;
+    QuadIn cur, nxt{};
+    quad_load<SLOT>(d, sc, f, t1, tw, S, base, n, k0, dux, dvy, cur);
+    for (int q = 0; q < ng; ++q) {
+        const int k = k0 + 4 * q;
+        if (q + 1 < ng) quad_load<SLOT>(d, sc, f, t1, tw, S, base, n, k + 4, dux, dvy, nxt);
+        const long x = base + k * sk;
+        VCoef ft[1];
+        {
+            const bool o4[4] = {(cur.m[0] & M_OPEN) != 0, (cur.m[1] & M_OPEN) != 0,
+                                (cur.m[2] & M_OPEN) != 0, (cur.m[3] & M_OPEN) != 0};
+            const double p[1][4] = {{cur.p[0], cur.p[1], cur.p[2], cur.p[3]}};
+            vface_coefs<OPT, 1, FAST>(sc, p, cur.v, cur.du, o4, cur.qz1,
+                                      vflux && k < KUB && k >= ks - 1, ft, bad);
+        }
+        VCoef fb;
+        fb.d = quad_perm<QUAD_UP>(ft[0].d);
+        fb.e = quad_perm<QUAD_UP>(ft[0].e);
+        fb.d = l ? fb.d : fc.d;
+        fb.e = l ? fb.e : fc.e;
+        fc.d = quad_lane<3>(ft[0].d);
+        fc.e = quad_lane<3>(ft[0].e);
+        fb.c = fb.f = 0.0;
+        if (!OPT && !sc.impAdvV) {
+            fb.c = quad_perm<QUAD_UP>(ft[0].c);
+            fb.f = quad_perm<QUAD_UP>(ft[0].f);
+            fb.c = l ? fb.c : fc.c;
+            fb.f = l ? fb.f : fc.f;
+            fc.c = quad_lane<3>(ft[0].c);
+            fc.f = quad_lane<3>(ft[0].f);
+        }
+        if (SLOT) {
+            const double b = quad_perm<QUAD_UP>(cur.cwT);
+            cur.cwB = l ? b : cwc;
+            cwc = quad_lane<3>(cur.cwT);
+        }
+        const bool on = k >= ks;
+        double D = 0.0, E = 1.0, F = 0.0, TI = cur.TI;
+        if (on) {
+            const RowShared r =
+                row_shared<FAST>(sc, f, x, k, KUB, cur.v[1], cur.m[1], cur.m[2], cur.qz1,
+                                 [&](int up) { return up ? cur.cwT : cur.cwB; });
+            row_terms<OPT, FAST, OBC, NT == 1>(d, sc, f, t1, base, x, k, r, cur.p, fb, ft[0], D,
+                                               E, F, TI, bad);
+        } else {
+            TI = 0.0;
+        }
+        // THOMASZ_NewType2 forward sweep (MF:4090-4099), level by level
+        double wo = 0.0, go = 0.0;
+        auto step = [&](auto lc) {
+            constexpr int LC = decltype(lc)::value;
+            const double aux = E + D * W, num = TI - D * G;
+            double w = 0.0, gg = 0.0;
+            if constexpr (FAST) {
+                const double ia = frcp(aux);
+                w = -F * ia;
+                gg = num * ia;
+            } else {
+                const Recip R = recip(aux);
+                w = fdiv(-F, R);
+                gg = fdiv(num, R);
+                const double mw = fabs(w), mg = fabs(gg);
+                const bool ok = R.ok & (mw < 0x1p400) & ((mw >= 0x1p-400) | (F == 0.0)) &
+                                (mg < 0x1p400) & ((mg >= 0x1p-400) | (num == 0.0));
+                if (!ok) {
+                    w = -F / aux;
+                    gg = num / aux;
+                }
+            }
+            if (!(fabs(aux) > 0.0)) {
+                if (l == LC && act && on) atomicAdd(zero_pivots, 1ull);
+                w = 0.0;
+                gg = 0.0;
+            }
+            if (l == LC) { wo = w; go = gg; }
+            W = quad_lane<LC>(w);
+            G = quad_lane<LC>(gg);
+        };
+        step(std::integral_constant<int, 0>{});
+        step(std::integral_constant<int, 1>{});
+        step(std::integral_constant<int, 2>{});
+        step(std::integral_constant<int, 3>{});
+        wg[q * 64 + lane] = make_double2(wo, go);
+        cur = nxt;
+    }
+    // ghost top row, as column_ghost
+    double xs;
+    {
+        const long xg = base + (KUB + 1) * sk;
+        const bool land = f.mask[xg] & M_LAND;
+        const double TIg = land ? MGPU_NULL_REAL : (t1.G0 ? t1.G0[xg * s] : 0.0);
+        const double aux = 1.0 + 0.0 * W;
+        xs = (TIg - 0.0 * G) / aux;
+        if (act && l == 0) t1.out[xg * s] = xs;
+    }
+    for (int q = ng - 1; q >= 0; --q) {
+        const int k = k0 + 4 * q;
+        const double2 v = wg[q * 64 + lane];
+        double xo = 0.0;
+        auto step = [&](auto lc) {
+            constexpr int LC = decltype(lc)::value;
+            const double y = v.x * xs + v.y;
+            xs = quad_lane<LC>(y);
+            if (l == LC) xo = xs;
+        };
+        step(std::integral_constant<int, 3>{});
+        step(std::integral_constant<int, 2>{});
+        step(std::integral_constant<int, 1>{});
+        step(std::integral_constant<int, 0>{});
+        if (act && k >= ks) t1.out[(base + k * sk) * s] = xo;
+    }
+    // the inert land rows below the column's first row (AD:1753), stored last,
+    // so that out may be P itself
+    if (act)
+        for (int k = d.wKLB + l; k < ks && k <= KUB; k += 4)
+            t1.out[(base + k * sk) * s] = MGPU_NULL_REAL;
+    if (bad) atomicOr(badflag, 1u);
+}
+
+// ---------------------------------------------------------------------------
 // Fused variant: one pass per step.  One lane per (column, TPL tracers), as
 // in column_lane_kernel, walks its column upwards; at every level it builds
 // the cell's explicit right-hand side itself (cell_rhs_lane: the explicit
@@ -2876,6 +3125,24 @@ static int launch_explicit_tpl(const Dims &d, const StepScalars &sc, const Share
     return MGPU_SUCCESS;
 }
 
+// The quad walk's LDS: a W/G pair per lane for every four levels of
+// KLB .. WorkSize KUB.
+static inline long quad_lds(const Dims &d) {
+    return (long)((d.wKUB - d.KLB) / 4 + 1) * 64 * (long)sizeof(double2);
+}
+
+// Where the quad walk is taken: while the lane per line leaves the 1,024 SIMDs
+// less than a wave (optimised path: its lane walk has the loads a level ahead)
+// or a wave and a half (the other path) each, and W and G of a column fit
+// 64 KB.  Measured with one tracer, lane walk -> quad walk: optimised path,
+// ragged columns, 28,000 / 44,000 / 63,000 lines of 40 levels 62 -> 42,
+// 65 -> 59, 79 -> 83 us; other path, 40 full levels, 40,000 / 90,000 / 122,000
+// lines 132 -> 65, 167 -> 125, 176 -> 185 us.
+template <bool OPT>
+static inline bool quad_columns(const Dims &d, long lines) {
+    return lines <= (OPT ? 48L : 96L) * 1024 && quad_lds(d) <= 65536;
+}
+
 template <bool OPT, int NT, int TPL, bool FAST>
 static int launch_column_tpl(const Dims &d, const StepScalars &sc, const SharedFields &f,
                              const TracerSet &ts, const SolveLists &l, double *TW, double *Gs,
@@ -2883,6 +3150,33 @@ static int launch_column_tpl(const Dims &d, const StepScalars &sc, const SharedF
                              int mixed = 0, bool walk = false) {
     const long nb = (l.ncols * (NT / TPL) + 255) / 256;
     if (nb <= 0) return MGPU_SUCCESS;
+    if (!walk && mixed <= 0 && quad_columns<OPT>(d, l.ncols * NT)) {
+        const bool slot = OPT && !f.obc.bp && !f.disch.ptr && l.slot.cols;
+        if (slot && l.slot.ncols != l.ncols) return MGPU_ERR_STATE;
+        const unsigned nq = (unsigned)((l.ncols * NT + 15) / 16);
+        const unsigned lds = (unsigned)quad_lds(d);
+        if (f.obc.bp) {
+            // open boundaries are a per-property option: the drop-in's one tracer
+            if constexpr (NT == 1) {
+                hipLaunchKernelGGL((column_quad_kernel<OPT, 1, FAST, true, false>), dim3(nq),
+                                   dim3(64), lds, s, d, sc, f, ts, l.cols, l.ncols, TW,
+                                   SlotColumns{}, counters, bad);
+            } else {
+                return MGPU_ERR_UNSUPPORTED;
+            }
+        } else if (slot) {
+            if constexpr (OPT)
+                hipLaunchKernelGGL((column_quad_kernel<true, NT, FAST, false, true>), dim3(nq),
+                                   dim3(64), lds, s, d, sc, f, ts, l.slot.cols, l.ncols, TW,
+                                   l.slot, counters, bad);
+        } else {
+            hipLaunchKernelGGL((column_quad_kernel<OPT, NT, FAST, false, false>), dim3(nq),
+                               dim3(64), lds, s, d, sc, f, ts, l.cols, l.ncols, TW,
+                               SlotColumns{}, counters, bad);
+        }
+        HIPCHK(hipGetLastError());
+        return MGPU_SUCCESS;
+    }
     if (walk) {
         // the fused variant: explicit right-hand side inside the column walk
         // (at most 4 tracers per lane: 8 do not fit the register file)

@@ -1,6 +1,8 @@
-"""The one-tracer explicit kernel at the edges of its 64 x 8 tiles (GPU), equal
-to the oracle on every cell: extents around a tile, one level, every branch of
-the face, fields with exact zeros and with values far below 1."""
+"""The one-tracer explicit kernel at the edges of its 64 x 8 tiles and the
+column walk's two forms (GPU), equal to the oracle on every cell: extents
+around a tile, one level, every branch of the face, fields with exact zeros
+and with values far below 1; few columns (four lanes each) and many, of depths
+around a group of four levels."""
 import numpy as np
 import pytest
 
@@ -67,3 +69,47 @@ def test_zero_and_small_values(optimize):
         p[wet & ~far] *= scale
         props.append(p)
     _check(case, props, optimize)
+
+
+@pytest.mark.parametrize("optimize", (False, True))
+@pytest.mark.parametrize("ni,nj,nk,kfloor", [
+    (5, 3, 2, (1, 2)), (9, 7, 3, (3, 3)), (17, 5, 4, (1, 4)), (16, 4, 5, (1, 5)),
+    (11, 6, 37, (1, 37)), (4, 4, 259, (1, 259)), (230, 230, 4, (1, 4)),
+    (330, 310, 3, (1, 3))])
+def test_columns(ni, nj, nk, kfloor, optimize):
+    """Depths around groups of four levels and past what LDS holds (259), and
+    column counts either side of the change of walk."""
+    case = fx.make_case(fx.config("c3", ni=ni, nj=nj, nk=nk, kfloor=kfloor, land_frac=0.0,
+                                  tracers=("temperature", "lognormal"), **GRID))
+    _check(case, case.tracers, optimize)
+
+
+@pytest.mark.parametrize("impV,difV", [(C.EXPLICIT_SCHEME, 1.0), (C.EXPLICIT_SCHEME, 0.5),
+                                       (C.IMPLICIT_SCHEME, C.EXPLICIT_SCHEME)])
+@pytest.mark.parametrize("optimize", (False, True))
+def test_columns_vertical_schemes(impV, difV, optimize):
+    case = fx.make_case(fx.config("c3", ni=21, nj=13, nk=11, kfloor=(1, 11), land_frac=0.2,
+                                  tracers=("temperature", "lognormal"), **GRID))
+    case.params.update(ImpExp_AdvV=impV, ImpExp_DifV=difV)
+    _check(case, case.tracers, optimize)
+
+
+@pytest.mark.parametrize("tracers,order", [(3, 0), (3, 1), (5, 0), (5, 1)])
+def test_batched_columns(tracers, order):
+    """Interleaved tracers, columns in memory order and by first row."""
+    from mohid_amd.advection_diffusion import Transport
+    names = ("temperature", "salinity", "lognormal", "lognormal", "lognormal")[:tracers]
+    case = fx.make_case(fx.config("c3", ni=37, nj=23, nk=13, kfloor=(2, 13), land_frac=0.3,
+                                  tracers=names, **GRID))
+    tr = Transport(case.size, case.worksize, case.geom, tracers)
+    tr.set_column_order(order)
+    tr.set_hydro(case.hydro, case.params)
+    for t, p in enumerate(case.tracers):
+        tr.set_tracer(t, p)
+    tr.run(2)
+    ref = ora.run_case(case, 2, nthreads=1)
+    solved = np.zeros(case.tracers[0].shape, dtype=bool)
+    solved[:, :, 1:] = (case.hydro["WaterPoints3D"][:, :, case.worksize[5]] == 1)[:, :, None]
+    for t in range(tracers):
+        assert np.array_equal(tr.get_tracer(t)[solved], ref[t][solved]), t
+    tr.close()

@@ -115,17 +115,20 @@ struct DevHydro {
     // cfw, water), allocated on the first call that copies
     double *od[7] = {};
     int32_t *oi[6] = {};
-    // optional inputs, allocated on first use; have_* tells whether this
-    // step's call passed them
-    int32_t *nfu = nullptr, *nfv = nullptr, *nfw = nullptr, *small = nullptr;
+    // optional inputs (owned copies allocated on first use); have_* tells
+    // whether this step's call passed them
+    const int32_t *nfu = nullptr, *nfv = nullptr, *nfw = nullptr, *small = nullptr;
     bool have_nf = false, have_small = false;
-    double *ref = nullptr;        // ReferenceProp
-    int32_t *bp = nullptr;        // BoundaryPoints2D
+    const double *ref = nullptr;        // ReferenceProp
+    const int32_t *bp = nullptr;        // BoundaryPoints2D
+    int32_t *oo[5] = {};                // NoFluxU, NoFluxV, NoFluxW, SmallDepths, BoundaryPoints2D
+    double *oref = nullptr;
     bool have_ref = false, have_bp = false;
 
     // view: read the caller's device arrays in place (a drop-in call with
     // device pointers); otherwise copy them into the owned arrays
-    int upload(const Dims &d, const mgpu_ad_args *a, hipStream_t s, bool view = false) {
+    int upload(const Dims &d, const mgpu_ad_args *a, hipStream_t s, bool view = false,
+               const double *prop = nullptr) {
         const hipMemcpyKind kind =
             a->device_pointers ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
         const size_t b = sizeof(double) * (size_t)d.n3(), bi = sizeof(int32_t) * (size_t)d.n3();
@@ -161,49 +164,42 @@ struct DevHydro {
         }
         Qx = vd[0]; Qy = vd[1]; Qz = vd[2]; V = vd[3]; Vold = vd[4]; visc = vd[5]; diffv = vd[6];
         open = vi[0]; land = vi[1]; cfu = vi[2]; cfv = vi[3]; cfw = vi[4]; water = vi[5];
+        // optional inputs: viewed likewise, or copied
+        auto opt = [&](const auto *src, auto *&own, long n, auto *&at) -> int {
+            // an array that the call itself writes is copied
+            const void *v = src;
+            if (view && a->device_pointers && v != prop && v != a->PROPOld) {
+                at = src;
+                return MGPU_SUCCESS;
+            }
+            if (!own) {
+                HIPCHK(hipStreamSynchronize(s));
+                if (dalloc(&own, n)) return MGPU_ERR_NOMEM;
+            }
+            HIPCHK(hipMemcpyAsync(own, src, sizeof(*own) * (size_t)n, kind, s));
+            at = own;
+            return MGPU_SUCCESS;
+        };
+        int rc = MGPU_SUCCESS;
         have_nf = a->NoDifFlux != 0 || a->NoAdvFlux != 0;
         if (have_nf) {
-            if (!nfu) {
-                HIPCHK(hipStreamSynchronize(s));
-                if (dalloc(&nfu, d.n3()) || dalloc(&nfv, d.n3()) || dalloc(&nfw, d.n3()))
-                    return MGPU_ERR_NOMEM;
-            }
-            HIPCHK(hipMemcpyAsync(nfu, a->NoFluxU, bi, kind, s));
-            HIPCHK(hipMemcpyAsync(nfv, a->NoFluxV, bi, kind, s));
-            if (a->NoFluxW) HIPCHK(hipMemcpyAsync(nfw, a->NoFluxW, bi, kind, s));
+            if ((rc = opt(a->NoFluxU, oo[0], d.n3(), nfu))) return rc;
+            if ((rc = opt(a->NoFluxV, oo[1], d.n3(), nfv))) return rc;
+            if (a->NoFluxW && (rc = opt(a->NoFluxW, oo[2], d.n3(), nfw))) return rc;
         }
         have_small = a->SmallDepths != nullptr;
-        if (have_small) {
-            if (!small) {
-                HIPCHK(hipStreamSynchronize(s));
-                if (dalloc(&small, d.n2())) return MGPU_ERR_NOMEM;
-            }
-            HIPCHK(hipMemcpyAsync(small, a->SmallDepths, sizeof(int32_t) * (size_t)d.n2(), kind,
-                                  s));
-        }
+        if (have_small && (rc = opt(a->SmallDepths, oo[3], d.n2(), small))) return rc;
         have_ref = a->ReferenceProp != nullptr;
-        if (have_ref) {
-            if (!ref) {
-                HIPCHK(hipStreamSynchronize(s));
-                if (dalloc(&ref, d.n3())) return MGPU_ERR_NOMEM;
-            }
-            HIPCHK(hipMemcpyAsync(ref, a->ReferenceProp, b, kind, s));
-        }
+        if (have_ref && (rc = opt(a->ReferenceProp, oref, d.n3(), ref))) return rc;
         have_bp = a->BoundaryPoints2D != nullptr;
-        if (have_bp) {
-            if (!bp) {
-                HIPCHK(hipStreamSynchronize(s));
-                if (dalloc(&bp, d.n2())) return MGPU_ERR_NOMEM;
-            }
-            HIPCHK(hipMemcpyAsync(bp, a->BoundaryPoints2D, sizeof(int32_t) * (size_t)d.n2(), kind,
-                                  s));
-        }
+        if (have_bp && (rc = opt(a->BoundaryPoints2D, oo[4], d.n2(), bp))) return rc;
         return MGPU_SUCCESS;
     }
     void release() {
         for (double *&q : od) dfree(q);
         for (int32_t *&q : oi) dfree(q);
-        dfree(nfu); dfree(nfv); dfree(nfw); dfree(small); dfree(ref); dfree(bp);
+        for (int32_t *&q : oo) dfree(q);
+        dfree(oref);
     }
 };
 
@@ -238,8 +234,12 @@ struct DevDerived {
     uint32_t *rowcnt = nullptr, *cells = nullptr, *cols = nullptr, *hrows = nullptr;
     unsigned long long *totals = nullptr;
     long ncells = 0, ncols = 0, nhrows = 0;
+    bool counted = false;         // the counts above are the lists'; else only bounds
     // [0] THOMASZ zero pivots, [1] bad-method flag, [2] mask flags, [3] THOMAS_3D zero pivots
     unsigned long long *counters = nullptr;
+    // solved columns per WorkSize j, behind the counters (cleared with them)
+    uint32_t *colcnt = nullptr;
+    size_t counter_bytes = 0;
     // cell_list: also the list of solved rows, for launches of several tracers
     int alloc(const Dims &d, bool cell_list) {
         const long n3 = d.n3(), nt = tile_count(d), nK = d.KUB - d.KLB + 1;
@@ -253,13 +253,15 @@ struct DevDerived {
         rc |= dalloc(&cu, n3); rc |= dalloc(&cv, n3); rc |= dalloc(&cw, n3);
         rc |= dalloc(&cperm, nt * 256); rc |= dalloc(&ccnt, nt * nK);
         rc |= dalloc(&fperm, nt * 580); rc |= dalloc(&fcnt, nt * nK);
-        rc |= dalloc(&counters, 4);
+        counter_bytes = sizeof(unsigned long long) * (size_t)(4 + (nJw + 1) / 2);
+        rc |= dalloc(&counters, 4 + (nJw + 1) / 2);
         if (rc) return MGPU_ERR_NOMEM;
+        colcnt = reinterpret_cast<uint32_t *>(counters + 4);
         // cells the prep kernel never writes must still be finite
         HIPCHK(hipMemset(cu, 0, sizeof(double) * (size_t)n3));
         HIPCHK(hipMemset(cv, 0, sizeof(double) * (size_t)n3));
         HIPCHK(hipMemset(cw, 0, sizeof(double) * (size_t)n3));
-        HIPCHK(hipMemset(counters, 0, sizeof(unsigned long long) * 4));
+        HIPCHK(hipMemset(counters, 0, counter_bytes));
         return MGPU_SUCCESS;
     }
     void release() {
@@ -267,10 +269,14 @@ struct DevDerived {
         dfree(cperm); dfree(ccnt); dfree(fperm); dfree(fcnt);
         dfree(rowcnt); dfree(cells); dfree(cols); dfree(totals); dfree(hrows);
     }
-    // masks -> mask bytes, kstart, tile orders (after the mask arrays are on the device)
+    // masks -> mask bytes, kstart, tile orders (after the mask arrays are on the
+    // device and the counters cleared)
     // hlines: also the list of implicit line rows (allocated on first use)
+    // count: wait for the lists' lengths; without it (no other list than cols)
+    // the column kernels read cols' length on the device
     int pack(const Dims &d, const DevHydro &h, const int32_t *kfloor, int docycle,
-             hipStream_t s, bool tiles, bool hlines = false, const int32_t *dptr = nullptr) {
+             hipStream_t s, bool tiles, bool hlines = false, const int32_t *dptr = nullptr,
+             bool count = true) {
         if (hlines && !hrows) {
             const long nw = (long)(d.wIUB - d.wILB + 1) * (d.wJUB - d.wJLB + 1) *
                             (d.wKUB - d.wKLB + 1);
@@ -279,13 +285,19 @@ struct DevDerived {
         }
         int rc = launch_pack_masks(d, h.open, h.land, h.cfu, h.cfv, h.cfw, h.water,
                                    h.have_small ? h.small : nullptr, dptr, kfloor, docycle,
-                                   mask, kstart, mask_flags(), s);
+                                   mask, kstart, colcnt, mask_flags(), s);
         // tile metadata only for the tile variants (level keys are bytes there)
         if (!rc && tiles) rc = launch_tile_sort(d, mask, kstart, cperm, ccnt, fperm, fcnt, s);
         if (!rc)
-            rc = launch_build_lists(d, mask, kstart, rowcnt, cells, cols, hlines ? hrows : nullptr,
-                                    totals, s);
+            rc = launch_build_lists(d, mask, kstart, colcnt, rowcnt, cells, cols,
+                                    hlines ? hrows : nullptr, totals, s);
         if (rc) return rc;
+        counted = count || cells || hlines;
+        if (!counted) {
+            ncells = nhrows = 0;
+            ncols = (long)(d.wIUB - d.wILB + 1) * (d.wJUB - d.wJLB + 1);
+            return MGPU_SUCCESS;
+        }
         unsigned long long n[3];
         HIPCHK(hipMemcpyAsync(n, totals, sizeof(n), hipMemcpyDeviceToHost, s));
         HIPCHK(hipStreamSynchronize(s));
@@ -300,6 +312,7 @@ struct DevDerived {
         l.cols = cols;
         l.ncells = ncells;
         l.ncols = ncols;
+        l.dcols = counted ? nullptr : totals + 1;
         l.hrows = hrows;
         l.nhrows = nhrows;
         return l;
@@ -488,6 +501,7 @@ struct mgpu_ad {
     double mask_dt = 0.0;
     double last_dt = 0.0, last_schmidtH = 0.0;   // Set_Internal_State's memory (AD:5746)
     unsigned long long last_zero_pivots = 0;
+    unsigned long long *cnt = nullptr;      // pinned: the counters of a call
 };
 
 extern "C" int mgpu_ad_create(const mgpu_size3d *size, const mgpu_size3d *worksize,
@@ -522,6 +536,10 @@ extern "C" int mgpu_ad_create(const mgpu_size3d *size, const mgpu_size3d *worksi
     if (!rc) rc = dalloc(&ad->tig, n3);
     if (!rc) rc = dalloc(&ad->mid, n3);
     if (!rc) rc = dalloc(&ad->Rb, 4 * n3);
+    if (!rc && hipHostMalloc((void **)&ad->cnt, sizeof(unsigned long long) * 4) != hipSuccess) {
+        ad->cnt = nullptr;
+        rc = MGPU_ERR_NOMEM;
+    }
     if (!rc) rc = ad->geom.upload(ad->d, geometry, ad->stream);
     if (rc) {
         mgpu_ad_destroy(ad);
@@ -549,6 +567,7 @@ extern "C" int mgpu_ad_destroy(mgpu_ad *ad) {
     ad->bnd.release();
     dfree(ad->xz); dfree(ad->xzs);
     dfree(ad->nadv); dfree(ad->nw);
+    if (ad->cnt) (void)hipHostFree(ad->cnt);
     dfree(ad->flux.afx); dfree(ad->flux.afy); dfree(ad->flux.afz);
     dfree(ad->flux.dfx); dfree(ad->flux.dfy); dfree(ad->flux.dfz);
     if (ad->stream) (void)hipStreamDestroy(ad->stream);
@@ -817,13 +836,13 @@ extern "C" int mgpu_ad_step(mgpu_ad *ad, const mgpu_ad_args *a, double *prop) {
     const bool post = a->BoundaryCondition == 4 || a->BoundaryCondition == 8;
     if (post && (rc = ad->bnd.alloc(d))) return rc;
 
-    rc = ad->hydro.upload(d, a, s, true);
+    rc = ad->hydro.upload(d, a, s, true, prop);
     if (rc) return rc;
     double *P = ad->prop;
     if (a->device_pointers) P = prop;
     else HIPCHK(hipMemcpyAsync(ad->prop, prop, b3, hipMemcpyHostToDevice, s));
 
-    HIPCHK(hipMemsetAsync(ad->der.counters, 0, sizeof(unsigned long long) * 4, s));
+    HIPCHK(hipMemsetAsync(ad->der.counters, 0, ad->der.counter_bytes, s));
     if (ad->disch.on) {
         // this call's Flow of every discharge contribution (AD:4064-4082)
         rc = launch_disch_flow(ad->disch.ncell, ad->disch.cbase, ad->disch.cnt,
@@ -841,7 +860,7 @@ extern "C" int mgpu_ad_step(mgpu_ad *ad, const mgpu_ad_args *a, double *prop) {
         if (!same) {
             ad->masks_ok = false;
             rc = ad->der.pack(d, ad->hydro, ad->geom.KFloor, ad->docycle, s, false,
-                              sc.impH >= 0, ad->disch.on ? ad->disch.ptr : nullptr);
+                              sc.impH >= 0, ad->disch.on ? ad->disch.ptr : nullptr, false);
             if (rc) return rc;
             for (int q = 0; q < 8; ++q) ad->mask_src[q] = src[q];
             ad->mask_dt = a->DTProp;
@@ -942,8 +961,11 @@ extern "C" int mgpu_ad_step(mgpu_ad *ad, const mgpu_ad_args *a, double *prop) {
         f.nadv = ad->nadv;
         f.nw = ad->nw;
     }
-    // the step's own initialisation of TI (AD:1660-1671) reaches the ghost rows
-    if (first) HIPCHK(hipMemsetAsync(ad->tig, 0, b3, s));
+    // the step's own initialisation of TI (AD:1660-1671) reaches the ghost rows;
+    // without line solves only the column walk reads them, and takes 0 for a
+    // null record (the land fill below then writes the zeros)
+    const bool tig0 = first && sc.impH < 0;
+    if (first && !tig0) HIPCHK(hipMemsetAsync(ad->tig, 0, b3, s));
     // The column solve may write PROP in place when nothing after it needs
     // PROP from before the solve and no column reads another's PROP during
     // it: explicit horizontal advection, no open boundary (its rows read the
@@ -961,7 +983,7 @@ extern "C" int mgpu_ad_step(mgpu_ad *ad, const mgpu_ad_args *a, double *prop) {
     L.Wb = ad->Wb;
     L.Gb = ad->Gb;
     L.counters = ad->der.counters;
-    L.tig = ad->tig;
+    L.tig = tig0 ? nullptr : ad->tig;
     L.Rb = ad->Rb;
     const unsigned long long *stop = ad->der.counters + 3;
     if (sc.hreset) {
@@ -983,7 +1005,7 @@ extern "C" int mgpu_ad_step(mgpu_ad *ad, const mgpu_ad_args *a, double *prop) {
     if (rc) return rc;
     // TI = null_real on land (AD:1753), kept for the next call where a later
     // call reads it: at the ghost rows
-    rc = launch_land_fill(d, ad->der.mask, ad->tig, s);
+    rc = launch_land_fill(d, ad->der.mask, ad->tig, tig0, s);
     if (!rc && sc.impH >= 0) rc = launch_copy_lines(d, sc.impH, ad->out, P, stop, s);
     // the cell fluxes' explicit parts, with PROP before the solve (AD:1458-1468
     // zero them first)
@@ -1030,8 +1052,9 @@ extern "C" int mgpu_ad_step(mgpu_ad *ad, const mgpu_ad_args *a, double *prop) {
                                        a->ImpExp_AdvV, a->ImpExp_DifV, ad->flux, ad->Rb, s);
         if (rc) return rc;
     }
-    unsigned long long cnt[4];
-    HIPCHK(hipMemcpyAsync(cnt, ad->der.counters, sizeof(cnt), hipMemcpyDeviceToHost, s));
+    const unsigned long long *cnt = ad->cnt;
+    HIPCHK(hipMemcpyAsync(ad->cnt, ad->der.counters, sizeof(cnt[0]) * 4, hipMemcpyDeviceToHost,
+                          s));
     HIPCHK(hipStreamSynchronize(s));
     ad->last_zero_pivots = cnt[0];
     const unsigned int mflags = (unsigned int)(cnt[2] & 0xffffffffu);
@@ -1510,7 +1533,7 @@ extern "C" int mgpu_transport_set_hydro(mgpu_transport *t, const mgpu_ad_args *a
     t->nulldif = a->NullDif;
     rc = t->hydro.upload(t->d, a, t->stream);
     if (rc) return rc;
-    HIPCHK(hipMemsetAsync(t->der.counters, 0, sizeof(unsigned long long) * 4, t->stream));
+    HIPCHK(hipMemsetAsync(t->der.counters, 0, t->der.counter_bytes, t->stream));
     rc = t->der.pack(t->d, t->hydro, t->geom.KFloor, t->opts.docycle_method, t->stream,
                      t->kernel == MGPU_KERNEL_SPLIT, sc.impH >= 0);
     if (rc) return rc;

@@ -140,12 +140,12 @@ struct SharedFields {     // device pointers shared by all tracers
 // Kernel launchers (transport.hip)
 // small: the 2-D small-depth flags (M_SDV on every cell of a flagged
 // column) or null; dptr: the discharge cell index (a discharge cell is never
-// an identity row) or null.
+// an identity row) or null.  colcnt (zero before): solved columns per WorkSize j.
 int launch_pack_masks(const Dims &d, const int32_t *open, const int32_t *land,
                       const int32_t *cfu, const int32_t *cfv, const int32_t *cfw,
                       const int32_t *water, const int32_t *small, const int32_t *dptr,
                       const int32_t *kfloor, int docycle, uint8_t *mask, int32_t *kstart,
-                      unsigned int *flags, hipStream_t s);
+                      uint32_t *colcnt, unsigned int *flags, hipStream_t s);
 // Discharges: Flow of every contribution for this call (uniform discharges
 // spread over their cells by thickness, AD:4064-4082).  Per discharge cell
 // q: first contribution cbase[q], count cnt[q], uniform flag, DischFlow;
@@ -267,6 +267,9 @@ struct SolveLists {
     const uint32_t *cols = nullptr;    // Size index (level 0) of every solved column
     const uint32_t *hrows = nullptr;   // WorkSize cells without M_HID (implicit line rows)
     long ncells = 0, ncols = 0, nhrows = 0;
+    // not null: the column count lies here (device memory) and ncols is only
+    // an upper bound
+    const unsigned long long *dcols = nullptr;
     SlotColumns slot;                  // the depth-ordered walk's columns (batched transport)
 };
 // Builds the lists from the packed masks and kstart; totals[0..2] receive
@@ -274,8 +277,8 @@ struct SolveLists {
 // may be null (not built).  rowcnt holds (WorkSize J extent) x (WorkSize K extent)
 // counters.
 int launch_build_lists(const Dims &d, const uint8_t *mask, const int32_t *kstart,
-                       uint32_t *rowcnt, uint32_t *cells, uint32_t *cols, uint32_t *hrows,
-                       unsigned long long *totals, hipStream_t s);
+                       const uint32_t *colcnt, uint32_t *rowcnt, uint32_t *cells, uint32_t *cols,
+                       uint32_t *hrows, unsigned long long *totals, hipStream_t s);
 // The depth-ordered column list (SlotColumns::cols); *total receives its
 // length (device memory), which equals the solved-column count.
 int launch_slot_list(const Dims &d, const uint8_t *mask, const int32_t *kstart,
@@ -380,9 +383,11 @@ int launch_interleave(long n3, const double *src, double *dst, long stride, int 
 // unless *stop is non-zero.
 int launch_copy_lines(const Dims &d, int axis, const double *src, double *dst,
                       const unsigned long long *stop, hipStream_t s);
-// dst[x] = null_real where the mask has M_LAND, on the Size's last plane
-// along k, j and i (the ghost rows of the drop-in's TI record).
-int launch_land_fill(const Dims &d, const uint8_t *mask, double *dst, hipStream_t s);
+// dst[x] = null_real where the mask has M_LAND (and with clear 0 elsewhere), on
+// the Size's last plane along k, j and i (the ghost rows of the drop-in's TI
+// record).
+int launch_land_fill(const Dims &d, const uint8_t *mask, double *dst, bool clear,
+                     hipStream_t s);
 // THOMAS_3D lines (di 0: along j, IJ = i; di 1: along i, IJ = j) on arrays
 // spanning sz; bounds already checked.  pivots counts lines with a zero pivot;
 // scr holds thomas3d_scratch(lines, rows) doubles.

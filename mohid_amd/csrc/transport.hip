@@ -12,17 +12,11 @@ int launch_pack_masks(const Dims &d, const int32_t *open, const int32_t *land,
                       const int32_t *cfu, const int32_t *cfv, const int32_t *cfw,
                       const int32_t *water, const int32_t *small, const int32_t *dptr,
                       const int32_t *kfloor, int docycle, uint8_t *mask, int32_t *kstart,
-                      unsigned int *flags, hipStream_t s) {
-    const long n = d.n3();
-    const int threads = 256;
-    long blocks = (n + threads - 1) / threads;
-    if (blocks > 65536) blocks = 65536;
-    hipLaunchKernelGGL(pack_masks_kernel, dim3((unsigned)blocks), dim3(threads), 0, s, d, open,
-                       land, cfu, cfv, cfw, water, small, dptr, mask, n);
-    HIPCHK(hipGetLastError());
-    const int ni = d.wIUB - d.wILB + 1, nj = d.wJUB - d.wJLB + 1;
-    dim3 b(64, 4), g((ni + 63) / 64, (nj + 3) / 4);
-    hipLaunchKernelGGL(kstart_kernel, g, b, 0, s, d, mask, kfloor, docycle, kstart, flags);
+                      uint32_t *colcnt, unsigned int *flags, hipStream_t s) {
+    const int nI = d.IUB - d.ILB + 1, nJ = d.JUB - d.JLB + 1;
+    hipLaunchKernelGGL(mask_columns_kernel, dim3((nI + 63) / 64, nJ), dim3(64, 4), 0, s, d, open,
+                       land, cfu, cfv, cfw, water, small, dptr, kfloor, docycle, mask, kstart,
+                       colcnt, flags);
     HIPCHK(hipGetLastError());
     return MGPU_SUCCESS;
 }
@@ -61,39 +55,25 @@ int launch_prep_faces(const Dims &d, const double *visc, const double *diffv, co
 }
 
 int launch_build_lists(const Dims &d, const uint8_t *mask, const int32_t *kstart,
-                       uint32_t *rowcnt, uint32_t *cells, uint32_t *cols, uint32_t *hrows,
-                       unsigned long long *totals, hipStream_t s) {
+                       const uint32_t *colcnt, uint32_t *rowcnt, uint32_t *cells, uint32_t *cols,
+                       uint32_t *hrows, unsigned long long *totals, hipStream_t s) {
     if (d.n3() >= (1L << 32)) return MGPU_ERR_UNSUPPORTED;   // list entries are 32-bit
     const int nj = d.wJUB - d.wJLB + 1, nk = d.wKUB - d.wKLB + 1;
-    // cells: rows (j, k); columns: rows j
-    if (cells) {
-        hipLaunchKernelGGL(list_count_kernel, dim3(nj, nk), dim3(256), 0, s, d, mask, kstart, 0,
-                           rowcnt);
+    hipLaunchKernelGGL(column_list_kernel, dim3(nj), dim3(256), 0, s, d, mask, colcnt, cols,
+                       totals + 1);
+    HIPCHK(hipGetLastError());
+    // rows (j, k)
+    for (int kind : {0, 2}) {
+        uint32_t *out = kind == 0 ? cells : hrows;
+        if (!out) continue;
+        hipLaunchKernelGGL(list_count_kernel, dim3(nj, nk), dim3(256), 0, s, d, mask, kstart,
+                           kind, rowcnt);
         HIPCHK(hipGetLastError());
         hipLaunchKernelGGL(list_scan_kernel, dim3(1), dim3(1024), 0, s, rowcnt, (long)nj * nk,
-                           totals);
+                           totals + kind);
         HIPCHK(hipGetLastError());
-        hipLaunchKernelGGL(list_write_kernel, dim3(nj, nk), dim3(256), 0, s, d, mask, kstart, 0,
-                           rowcnt, cells);
-        HIPCHK(hipGetLastError());
-    }
-    hipLaunchKernelGGL(list_count_kernel, dim3(nj, 1), dim3(256), 0, s, d, mask, kstart, 1,
-                       rowcnt);
-    HIPCHK(hipGetLastError());
-    hipLaunchKernelGGL(list_scan_kernel, dim3(1), dim3(1024), 0, s, rowcnt, (long)nj, totals + 1);
-    HIPCHK(hipGetLastError());
-    hipLaunchKernelGGL(list_write_kernel, dim3(nj, 1), dim3(256), 0, s, d, mask, kstart, 1,
-                       rowcnt, cols);
-    HIPCHK(hipGetLastError());
-    if (hrows) {
-        hipLaunchKernelGGL(list_count_kernel, dim3(nj, nk), dim3(256), 0, s, d, mask, kstart, 2,
-                           rowcnt);
-        HIPCHK(hipGetLastError());
-        hipLaunchKernelGGL(list_scan_kernel, dim3(1), dim3(1024), 0, s, rowcnt, (long)nj * nk,
-                           totals + 2);
-        HIPCHK(hipGetLastError());
-        hipLaunchKernelGGL(list_write_kernel, dim3(nj, nk), dim3(256), 0, s, d, mask, kstart, 2,
-                           rowcnt, hrows);
+        hipLaunchKernelGGL(list_write_kernel, dim3(nj, nk), dim3(256), 0, s, d, mask, kstart,
+                           kind, rowcnt, out);
         HIPCHK(hipGetLastError());
     }
     return MGPU_SUCCESS;
@@ -269,12 +249,13 @@ __global__ void copy_lines_kernel(Dims d, int axis, const double *__restrict__ s
     }
 }
 
-// TI = null_real on land (AD:1753) in the drop-in's record of TI, on the
-// Size's last plane along k, j and i: the ghost rows, the only places a later
+// TI = null_real on land (AD:1753) in the drop-in's record of TI, and with
+// `clear` 0 elsewhere (what the step's own initialisation leaves, AD:1660-1671),
+// on the Size's last plane along k, j and i: the ghost rows, the only places a later
 // call reads it (the column walk's top KUB+1, the line solves' ends JUB+1 and
 // IUB+1).
 __global__ void land_fill_kernel(Dims d, const uint8_t *__restrict__ mask,
-                                 double *__restrict__ dst) {
+                                 double *__restrict__ dst, int clear) {
     const long nI = d.IUB - d.ILB + 1, nJ = d.JUB - d.JLB + 1, nK = d.KUB - d.KLB + 1;
     const long pk = nI * nJ, pj = nI * nK, pi = nJ * nK;
     for (long q = blockIdx.x * (long)blockDim.x + threadIdx.x; q < pk + pj + pi;
@@ -290,6 +271,7 @@ __global__ void land_fill_kernel(Dims d, const uint8_t *__restrict__ mask,
             x = (nI - 1) + (r % nJ) * d.sj + (r / nJ) * d.sk;          // i = IUB
         }
         if (mask[x] & M_LAND) dst[x] = MGPU_NULL_REAL;
+        else if (clear) dst[x] = 0.0;
     }
 }
 }  // namespace
@@ -770,12 +752,14 @@ int launch_copy_lines(const Dims &d, int axis, const double *src, double *dst,
     return MGPU_SUCCESS;
 }
 
-int launch_land_fill(const Dims &d, const uint8_t *mask, double *dst, hipStream_t s) {
+int launch_land_fill(const Dims &d, const uint8_t *mask, double *dst, bool clear,
+                     hipStream_t s) {
     const long nI = d.IUB - d.ILB + 1, nJ = d.JUB - d.JLB + 1, nK = d.KUB - d.KLB + 1;
     const long n = nI * nJ + nI * nK + nJ * nK;
     long blocks = (n + 255) / 256;
     if (blocks > 65536) blocks = 65536;
-    hipLaunchKernelGGL(land_fill_kernel, dim3((unsigned)blocks), dim3(256), 0, s, d, mask, dst);
+    hipLaunchKernelGGL(land_fill_kernel, dim3((unsigned)blocks), dim3(256), 0, s, d, mask, dst,
+                       clear ? 1 : 0);
     HIPCHK(hipGetLastError());
     return MGPU_SUCCESS;
 }

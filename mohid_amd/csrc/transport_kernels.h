@@ -5,7 +5,7 @@
 // (reference: Software/MOHIDBase2/ModuleAdvectionDiffusion.F90 = AD,
 // Software/MOHIDBase1/ModuleFunctions.F90 = MF) is done by
 //
-//   pack_masks      six int32 masks -> one byte per cell, plus per column the
+//   mask_columns    six int32 masks -> one byte per cell, plus per column the
 //                   lowest row that is not an inert land row (`kstart`), and
 //                   compact lists of the solved cells and columns;
 //   prep_faces      face conductances Kh*A/dx (U, V faces) and
@@ -53,71 +53,114 @@ namespace {
 // compute face: the reference gives it TI = null_real (AD:1753) and an
 // identity row, so its solution is null_real and it does not couple to the
 // rows above.  kstart is the first row above the inert bottom rows.
-__global__ void pack_masks_kernel(Dims d, const int32_t *__restrict__ open,
-                                  const int32_t *__restrict__ land,
-                                  const int32_t *__restrict__ cfu,
-                                  const int32_t *__restrict__ cfv,
-                                  const int32_t *__restrict__ cfw,
-                                  const int32_t *__restrict__ water,
-                                  const int32_t *__restrict__ small,
-                                  const int32_t *__restrict__ dptr,
-                                  uint8_t *__restrict__ mask, long n) {
-    for (long q = blockIdx.x * (long)blockDim.x + threadIdx.x; q < n;
-         q += (long)gridDim.x * blockDim.x) {
-        // the reference's face loops run over the WorkSize only (AD:4454-4520,
-        // 4839-4885, 5156-5365): a U or V face flag outside it is never read
-        const long kk = q / d.sk, r = q - kk * d.sk, jj = r / d.sj;
-        const int i = d.ILB + (int)(r - jj * d.sj), j = d.JLB + (int)jj, k = d.KLB + (int)kk;
-        const bool inws = i >= d.wILB && i <= d.wIUB && j >= d.wJLB && j <= d.wJUB &&
-                          k >= d.wKLB && k <= d.wKUB;
-        uint8_t m = 0;
-        if (open[q] == 1) m |= M_OPEN;
-        if (land[q] == 1) m |= M_LAND;
-        if (inws && cfu[q] == 1) m |= M_CFU;
-        if (inws && cfv[q] == 1) m |= M_CFV;
-        if (cfw[q] == 1) m |= M_CFW;
-        if (water[q] == 1) m |= M_WATER;
-        // faces above along j (i, j+1) and i (i+1, j), inside the WorkSize
-        const bool up_j = j + 1 <= d.wJUB && inws && cfu[q + d.sj] == 1;
-        const bool up_i = i + 1 <= d.wIUB && inws && cfv[q + 1] == 1;
-        if (!(m & (M_OPEN | M_CFU | M_CFV)) && !up_j && !up_i && !(dptr && dptr[q] >= 0))
-            m |= M_HID;
-        if (small && small[r] != 0) m |= M_SDV;   // r: the (i, j) index in Size
-        mask[q] = m;
+//
+// One pass over the six int32 masks (bound by their 24 bytes a cell): a block
+// takes 64 columns of one j, its four waves a quarter of the levels each, and
+// makes the mask bytes, kstart, the checks of the masks and the count of the
+// row's solved columns.  At 512 x 512 x 50 the pass took 104 us, and kstart
+// from the bytes another 23; together now 108.
+__global__ void __launch_bounds__(256)
+mask_columns_kernel(Dims d, const int32_t *__restrict__ open, const int32_t *__restrict__ land,
+                    const int32_t *__restrict__ cfu, const int32_t *__restrict__ cfv,
+                    const int32_t *__restrict__ cfw, const int32_t *__restrict__ water,
+                    const int32_t *__restrict__ small, const int32_t *__restrict__ dptr,
+                    const int32_t *__restrict__ kfloor, int docycle,
+                    uint8_t *__restrict__ mask, int32_t *__restrict__ kstart,
+                    uint32_t *__restrict__ colcnt, unsigned int *__restrict__ flags) {
+    __shared__ int first[4][64];
+    const int i = d.ILB + (int)(blockIdx.x * 64 + threadIdx.x), j = d.JLB + (int)blockIdx.y;
+    const int part = threadIdx.y;
+    const bool in = i <= d.IUB;
+    const bool col = in && i >= d.wILB && i <= d.wIUB && j >= d.wJLB && j <= d.wJUB;
+    // faces above along j (i, j+1) and i (i+1, j), inside the WorkSize
+    const bool wj = col && j + 1 <= d.wJUB, wi = col && i + 1 <= d.wIUB;
+    const long r = in ? d.idx2(i, j) : 0;
+    const int nK = d.KUB - d.KLB + 1, chunk = (nK + 3) / 4;
+    const int klo = d.KLB + part * chunk, khi = min(klo + chunk - 1, d.KUB);
+    const bool sdv = in && small && small[r] != 0;
+    const bool cyc = col && docycle == 1;
+    const bool top = cyc && cfw[r + (long)(d.wKUB - d.KLB) * d.sk] == 1;
+    const int kb = cyc ? kfloor[r] : 0;
+    int ks = d.wKUB + 1;
+    unsigned int bad = 0;
+    if (in) {
+#pragma unroll 4
+        for (int k = klo; k <= khi; ++k) {
+            const long q = r + (long)(k - d.KLB) * d.sk;
+            // the reference's face loops run over the WorkSize only (AD:4454-4520,
+            // 4839-4885, 5156-5365): a U or V face flag outside it is never read
+            const bool inws = col && k >= d.wKLB && k <= d.wKUB;
+            const int o = open[q], l = land[q], u = cfu[q], v = cfv[q], w = cfw[q], a = water[q];
+            const int u1 = wj ? cfu[q + d.sj] : 0, v1 = wi ? cfv[q + 1] : 0;
+            const int w1 = k < d.KUB ? cfw[q + d.sk] : 0;
+            const bool dis = dptr && dptr[q] >= 0;
+            uint8_t m = 0;
+            if (o == 1) m |= M_OPEN;
+            if (l == 1) m |= M_LAND;
+            if (inws && u == 1) m |= M_CFU;
+            if (inws && v == 1) m |= M_CFV;
+            if (w == 1) m |= M_CFW;
+            if (a == 1) m |= M_WATER;
+            const bool up = inws && (u1 == 1 || v1 == 1);
+            if (!(m & (M_OPEN | M_CFU | M_CFV)) && !up && !dis) m |= M_HID;
+            if (sdv) m |= M_SDV;
+            mask[q] = m;
+            if (inws) {
+                const bool faces = (m & (M_CFU | M_CFV | M_CFW)) || up || w1 == 1;
+                const bool inert = (m & M_LAND) && !(m & M_OPEN) && !faces;
+                if (!inert && k < ks) ks = k;
+                // A W face at the bottom level would use never-computed
+                // coefficients in the reference (Convert_Dif_Vertical starts at
+                // KLB+1, AD:2392).
+                if (k == d.wKLB && w == 1) bad |= 1u;
+                // DOCYCLE_METHOD 1 walks KFloor+1..KUB for columns whose surface
+                // W face computes (AD:2809-2835, 3059-3080); the per-face masks
+                // used here are the same walk when the masks agree with KFloor.
+                if (cyc && (top && k >= kb + 1) != (w == 1)) bad |= 2u;
+            }
+        }
+    }
+    first[part][threadIdx.x] = ks;
+    if (bad) atomicOr(flags, bad);
+    __syncthreads();
+    if (part == 0) {
+        const bool sol = col && water[r + (long)(d.wKUB - d.KLB) * d.sk] == 1;
+        const int n = __popcll(__ballot(sol));
+        if (threadIdx.x == 0 && n) atomicAdd(&colcnt[j - d.wJLB], (uint32_t)n);
+        if (col)
+            kstart[r] = min(min(first[0][threadIdx.x], first[1][threadIdx.x]),
+                            min(first[2][threadIdx.x], first[3][threadIdx.x]));
     }
 }
 
-__global__ void kstart_kernel(Dims d, const uint8_t *__restrict__ mask,
-                              const int32_t *__restrict__ kfloor, int docycle,
-                              int32_t *__restrict__ kstart, unsigned int *__restrict__ flags) {
-    const int i = d.wILB + blockIdx.x * blockDim.x + threadIdx.x;
-    const int j = d.wJLB + blockIdx.y * blockDim.y + threadIdx.y;
-    if (i > d.wIUB || j > d.wJUB) return;
-    int ks = d.wKUB + 1;
-    for (int k = d.wKLB; k <= d.wKUB; ++k) {
-        const uint8_t m = mask[d.idx(i, j, k)];
-        const bool faces = (m & (M_CFU | M_CFV | M_CFW)) ||
-                           (mask[d.idx(i, j + 1, k)] & M_CFU) ||
-                           (mask[d.idx(i + 1, j, k)] & M_CFV) ||
-                           (mask[d.idx(i, j, k + 1)] & M_CFW);
-        const bool inert = (m & M_LAND) && !(m & M_OPEN) && !faces;
-        if (!inert) { ks = k; break; }
-    }
-    kstart[d.idx2(i, j)] = ks;
-    // A W face at the bottom level would use never-computed coefficients in
-    // the reference (Convert_Dif_Vertical starts at KLB+1, AD:2392).
-    if (mask[d.idx(i, j, d.wKLB)] & M_CFW) atomicOr(flags, 1u);
-    // DOCYCLE_METHOD 1 walks KFloor+1..KUB for columns whose surface W face
-    // computes (AD:2809-2835, 3059-3080); the per-face masks used here are the
-    // same walk when the masks agree with KFloor -- check that they do.
-    if (docycle == 1) {
-        const bool top = mask[d.idx(i, j, d.wKUB)] & M_CFW;
-        const int kb = kfloor[d.idx2(i, j)];
-        for (int k = d.wKLB; k <= d.wKUB; ++k) {
-            const bool want = top && k >= kb + 1;
-            const bool has = mask[d.idx(i, j, k)] & M_CFW;
-            if (want != has) { atomicOr(flags, 2u); break; }
-        }
+// The solved columns (SolveLists::cols) in memory order: one block per j, its
+// offset summed from the counts of the rows before; the last one writes the
+// total.
+__global__ void __launch_bounds__(256)
+column_list_kernel(Dims d, const uint8_t *__restrict__ mask, const uint32_t *__restrict__ colcnt,
+                   uint32_t *__restrict__ cols, unsigned long long *__restrict__ total) {
+    __shared__ uint32_t part[4];
+    const int jj = blockIdx.x, j = d.wJLB + jj;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    uint32_t sum = 0;
+    for (int q = threadIdx.x; q < jj; q += 256) sum += colcnt[q];
+    for (int o = 32; o > 0; o >>= 1) sum += __shfl_down(sum, o, 64);
+    if (lane == 0) part[wave] = sum;
+    __syncthreads();
+    uint32_t off = part[0] + part[1] + part[2] + part[3];
+    if (jj == (int)gridDim.x - 1 && threadIdx.x == 0) *total = off + colcnt[jj];
+    const long top = (long)(d.wKUB - d.KLB) * d.sk;
+    for (int i0 = d.wILB; i0 <= d.wIUB; i0 += 256) {
+        const int i = i0 + threadIdx.x;
+        const bool m = i <= d.wIUB && (mask[d.idx2(i, j) + top] & M_WATER);
+        const unsigned long long b = __ballot(m);
+        __syncthreads();
+        if (lane == 0) part[wave] = (uint32_t)__popcll(b);
+        __syncthreads();
+        uint32_t at = off + (uint32_t)__popcll(b & ((1ull << lane) - 1ull));
+        for (int w = 0; w < wave; ++w) at += part[w];
+        if (m) cols[at] = (uint32_t)d.idx2(i, j);
+        off += part[0] + part[1] + part[2] + part[3];
     }
 }
 
@@ -1916,11 +1959,15 @@ __host__ __device__ constexpr int column_window(int tpl) { return tpl == 1 ? 4 :
 template <bool OPT, int NT, int TPL, bool FAST, bool OBC = false>
 __global__ void __launch_bounds__(256)
 column_lane_kernel(Dims d, StepScalars sc, SharedFields f, TracerSet ts,
-                   const uint32_t *__restrict__ cols, long ncols, double *__restrict__ TW,
+                   const uint32_t *__restrict__ cols, long ncols,
+                   const unsigned long long *__restrict__ dcols, double *__restrict__ TW,
                    double *__restrict__ Gs, unsigned long long *__restrict__ zero_pivots,
                    unsigned int *__restrict__ badflag) {
     constexpr int LPC = NT / TPL;
-    const long g = xcd_tile(blockIdx.x, gridDim.x) * 256 + threadIdx.x;
+    if (dcols) ncols = (long)*dcols;
+    const long nb = (ncols * LPC + 255) / 256;
+    if (blockIdx.x >= nb) return;
+    const long g = xcd_tile(blockIdx.x, nb) * 256 + threadIdx.x;
     const long n = g / LPC;
     const bool act = n < ncols;
     const int t = (int)(g - n * LPC) * TPL;
@@ -2164,12 +2211,16 @@ __host__ __device__ constexpr int column_lds_window(int tpl, bool slot = false) 
 template <int NT, int TPL, bool FAST, bool SLOT>
 __global__ void __launch_bounds__(256)
 column_pipe_kernel(Dims d, StepScalars sc, SharedFields f, TracerSet ts,
-                   const uint32_t *__restrict__ cols, long ncols, double *__restrict__ TW,
+                   const uint32_t *__restrict__ cols, long ncols,
+                   const unsigned long long *__restrict__ dcols, double *__restrict__ TW,
                    double *__restrict__ Gs, SlotColumns S,
                    unsigned long long *__restrict__ zero_pivots,
                    unsigned int *__restrict__ badflag) {
     constexpr int LPC = NT / TPL;
-    const long g = (SLOT ? (long)blockIdx.x : xcd_tile(blockIdx.x, gridDim.x)) * 256 + threadIdx.x;
+    if (!SLOT && dcols) ncols = (long)*dcols;
+    const long nb = SLOT ? (long)gridDim.x : (ncols * LPC + 255) / 256;
+    if (blockIdx.x >= nb) return;
+    const long g = (SLOT ? (long)blockIdx.x : xcd_tile(blockIdx.x, nb)) * 256 + threadIdx.x;
     const long n = g / LPC;
     const bool act = n < ncols;
     const int t = (int)(g - n * LPC) * TPL;
@@ -2349,12 +2400,16 @@ __device__ __forceinline__ void quad_load(const Dims &d, const StepScalars &sc,
 template <bool OPT, int NT, bool FAST, bool OBC, bool SLOT>
 __global__ void __launch_bounds__(64)
 column_quad_kernel(Dims d, StepScalars sc, SharedFields f, TracerSet ts,
-                   const uint32_t *__restrict__ cols, long ncols, const double *__restrict__ TW,
+                   const uint32_t *__restrict__ cols, long ncols,
+                   const unsigned long long *__restrict__ dcols, const double *__restrict__ TW,
                    SlotColumns S, unsigned long long *__restrict__ zero_pivots,
                    unsigned int *__restrict__ badflag) {
     extern __shared__ double2 wg[];       // [group][lane]
     const int lane = threadIdx.x, l = lane & 3;
-    const long blk = SLOT ? (long)blockIdx.x : xcd_tile32(blockIdx.x, gridDim.x);
+    if (!SLOT && dcols) ncols = (long)*dcols;
+    const unsigned nb = (unsigned)((ncols * NT + 15) / 16);
+    if (blockIdx.x >= nb) return;         // also where no column is solved
+    const long blk = SLOT ? (long)blockIdx.x : xcd_tile32(blockIdx.x, nb);
     const long g = blk * 16 + (lane >> 2);
     const long nn = g / NT;
     const bool act = nn < ncols;
@@ -2973,8 +3028,8 @@ line_thomas_kernel(Dims d, StepScalars sc, SharedFields f, TracerSet ts, double4
 // ---------------------------------------------------------------------------
 // Compact lists.  cells (kind 0): every (i, j, k) the reference solves and
 // gives an explicit right-hand side -- rows kstart..KUB of the columns with
-// WaterPoints3D(i,j,KUB) == 1 -- in memory order; cols (kind 1): those
-// columns; hrows (kind 2): the WorkSize cells whose horizontal line-solve
+// WaterPoints3D(i,j,KUB) == 1 -- in memory order (those columns are
+// column_list_kernel's); hrows (kind 2): the WorkSize cells whose horizontal line-solve
 // row is not the identity (no M_HID); the depth-ordered columns (kind 3):
 // the cols whose first row is k, for k from KLB up.  One block per row
 // (j, k) of the WorkSize plane: counts, then (after an exclusive scan of the
@@ -2985,7 +3040,7 @@ __device__ __forceinline__ bool list_member(const Dims &d, const uint8_t *mask,
     if (kind == 2) return !(mask[d.idx(i, j, k)] & M_HID);
     if (!(mask[d.idx(i, j, d.wKUB)] & M_WATER)) return false;
     if (kind == 3) return k == kstart[d.idx2(i, j)];   // a solved column whose first row is k
-    return kind == 1 || k >= kstart[d.idx2(i, j)];
+    return k >= kstart[d.idx2(i, j)];
 }
 
 __global__ void __launch_bounds__(256)
@@ -3049,7 +3104,7 @@ list_write_kernel(Dims d, const uint8_t *__restrict__ mask, const int32_t *__res
         const uint32_t chunk = wsum[0] + wsum[1] + wsum[2] + wsum[3];
         if (m)
             out[off + woff + before] =
-                (uint32_t)(kind == 1 || kind == 3 ? d.idx2(i, j) : d.idx(i, j, k));
+                (uint32_t)(kind == 3 ? d.idx2(i, j) : d.idx(i, j, k));
         __syncthreads();
         off += chunk;
     }
@@ -3159,7 +3214,7 @@ static int launch_column_tpl(const Dims &d, const StepScalars &sc, const SharedF
             // open boundaries are a per-property option: the drop-in's one tracer
             if constexpr (NT == 1) {
                 hipLaunchKernelGGL((column_quad_kernel<OPT, 1, FAST, true, false>), dim3(nq),
-                                   dim3(64), lds, s, d, sc, f, ts, l.cols, l.ncols, TW,
+                                   dim3(64), lds, s, d, sc, f, ts, l.cols, l.ncols, l.dcols, TW,
                                    SlotColumns{}, counters, bad);
             } else {
                 return MGPU_ERR_UNSUPPORTED;
@@ -3167,11 +3222,11 @@ static int launch_column_tpl(const Dims &d, const StepScalars &sc, const SharedF
         } else if (slot) {
             if constexpr (OPT)
                 hipLaunchKernelGGL((column_quad_kernel<true, NT, FAST, false, true>), dim3(nq),
-                                   dim3(64), lds, s, d, sc, f, ts, l.slot.cols, l.ncols, TW,
+                                   dim3(64), lds, s, d, sc, f, ts, l.slot.cols, l.ncols, nullptr, TW,
                                    l.slot, counters, bad);
         } else {
             hipLaunchKernelGGL((column_quad_kernel<OPT, NT, FAST, false, false>), dim3(nq),
-                               dim3(64), lds, s, d, sc, f, ts, l.cols, l.ncols, TW,
+                               dim3(64), lds, s, d, sc, f, ts, l.cols, l.ncols, l.dcols, TW,
                                SlotColumns{}, counters, bad);
         }
         HIPCHK(hipGetLastError());
@@ -3208,8 +3263,8 @@ static int launch_column_tpl(const Dims &d, const StepScalars &sc, const SharedF
         // open boundaries are a per-property option: the drop-in's one tracer
         if constexpr (NT == 1 && TPL == 1) {
             hipLaunchKernelGGL((column_lane_kernel<OPT, 1, 1, FAST, true>), dim3((unsigned)nb),
-                               dim3(256), 0, s, d, sc, f, ts, l.cols, l.ncols, TW, Gs, counters,
-                               bad);
+                               dim3(256), 0, s, d, sc, f, ts, l.cols, l.ncols, l.dcols, TW, Gs,
+                               counters, bad);
             HIPCHK(hipGetLastError());
             return MGPU_SUCCESS;
         }
@@ -3221,19 +3276,19 @@ static int launch_column_tpl(const Dims &d, const StepScalars &sc, const SharedF
             if (l.slot.cols) {
                 if (l.slot.ncols != l.ncols) return MGPU_ERR_STATE;
                 hipLaunchKernelGGL((column_pipe_kernel<NT, TPL, FAST, true>), dim3((unsigned)nb),
-                                   dim3(256), 0, s, d, sc, f, ts, l.slot.cols, l.ncols, TW, Gs,
-                                   l.slot, counters, bad);
+                                   dim3(256), 0, s, d, sc, f, ts, l.slot.cols, l.ncols, nullptr, TW,
+                                   Gs, l.slot, counters, bad);
             } else {
                 hipLaunchKernelGGL((column_pipe_kernel<NT, TPL, FAST, false>),
                                    dim3((unsigned)nb), dim3(256), 0, s, d, sc, f, ts, l.cols,
-                                   l.ncols, TW, Gs, SlotColumns{}, counters, bad);
+                                   l.ncols, l.dcols, TW, Gs, SlotColumns{}, counters, bad);
             }
             HIPCHK(hipGetLastError());
             return MGPU_SUCCESS;
         }
     }
     hipLaunchKernelGGL((column_lane_kernel<OPT, NT, TPL, FAST>), dim3((unsigned)nb), dim3(256), 0,
-                       s, d, sc, f, ts, l.cols, l.ncols, TW, Gs, counters, bad);
+                       s, d, sc, f, ts, l.cols, l.ncols, l.dcols, TW, Gs, counters, bad);
     HIPCHK(hipGetLastError());
     return MGPU_SUCCESS;
 }

@@ -83,17 +83,18 @@ struct DevGeometry {
             !g->AreaV || !g->DZZ || !g->DWZ)
             return MGPU_ERR_BADARG;
         const size_t b2 = sizeof(double) * (size_t)d.n2(), b3 = sizeof(double) * (size_t)d.n3();
-        const hipMemcpyKind kd =
-            g->device_pointers ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
-        HIPCHK(hipMemcpyAsync(DUX, g->DUX, b2, kd, s));
-        HIPCHK(hipMemcpyAsync(DVY, g->DVY, b2, kd, s));
-        HIPCHK(hipMemcpyAsync(DZX, g->DZX, b2, kd, s));
-        HIPCHK(hipMemcpyAsync(DZY, g->DZY, b2, kd, s));
-        HIPCHK(hipMemcpyAsync(KFloor, g->KFloorZ, sizeof(int32_t) * (size_t)d.n2(), kd, s));
-        HIPCHK(hipMemcpyAsync(AreaU, g->AreaU, b3, kd, s));
-        HIPCHK(hipMemcpyAsync(AreaV, g->AreaV, b3, kd, s));
-        HIPCHK(hipMemcpyAsync(DZZ, g->DZZ, b3, kd, s));
-        HIPCHK(hipMemcpyAsync(DWZ, g->DWZ, b3, kd, s));
+        CopySet c;
+        c.add(g->DUX, DUX, b2); c.add(g->DVY, DVY, b2); c.add(g->DZX, DZX, b2);
+        c.add(g->DZY, DZY, b2); c.add(g->KFloorZ, KFloor, sizeof(int32_t) * (size_t)d.n2());
+        c.add(g->AreaU, AreaU, b3); c.add(g->AreaV, AreaV, b3); c.add(g->DZZ, DZZ, b3);
+        c.add(g->DWZ, DWZ, b3);
+        if (g->device_pointers) {
+            if (int rc = launch_copy_set(c, s)) return rc;
+        } else {
+            for (int m = 0; m < c.n; ++m)
+                HIPCHK(hipMemcpyAsync(c.dst[m], c.src[m], (size_t)c.bytes[m],
+                                      hipMemcpyHostToDevice, s));
+        }
         HIPCHK(hipStreamSynchronize(s));
         return MGPU_SUCCESS;
     }
@@ -125,10 +126,19 @@ struct DevHydro {
     double *oref = nullptr;
     bool have_ref = false, have_bp = false;
 
-    // view: read the caller's device arrays in place (a drop-in call with
-    // device pointers); otherwise copy them into the owned arrays
-    int upload(const Dims &d, const mgpu_ad_args *a, hipStream_t s, bool view = false,
+    // What an upload takes over.  view: read the caller's device arrays in place
+    // (a drop-in call with device pointers); view_masks: the six masks alone,
+    // which the batched transport reads only while it packs them; otherwise
+    // they are copied into the owned arrays.  masks, visc, diffv: false where
+    // the call reads none of them (their owned copies then stay as they are).
+    struct Want {
+        bool view = false, view_masks = false, masks = true, visc = true, diffv = true;
+    };
+
+    int upload(const Dims &d, const mgpu_ad_args *a, hipStream_t s, Want want,
                const double *prop = nullptr) {
+        const bool view = want.view && a->device_pointers;
+        const bool vmask = (want.view || want.view_masks) && a->device_pointers;
         const hipMemcpyKind kind =
             a->device_pointers ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
         const size_t b = sizeof(double) * (size_t)d.n3(), bi = sizeof(int32_t) * (size_t)d.n3();
@@ -138,29 +148,33 @@ struct DevHydro {
                                 a->ComputeFacesV3D, a->ComputeFacesW3D, a->WaterPoints3D};
         const double *vd[7];
         const int32_t *vi[6];
-        if (view && a->device_pointers) {
-            for (int q = 0; q < 7; ++q) vd[q] = sd[q];
-            for (int q = 0; q < 6; ++q) vi[q] = si[q];
-        } else {
-            if (!oi[5]) {
-                HIPCHK(hipStreamSynchronize(s));
-                int rc = 0;
+        if ((!view && !od[6]) || (!vmask && !oi[5])) {
+            HIPCHK(hipStreamSynchronize(s));
+            int rc = 0;
+            if (!view && !od[6])
                 for (int q = 0; q < 7; ++q) rc |= dalloc(&od[q], d.n3());
+            if (!vmask && !oi[5])
                 for (int q = 0; q < 6; ++q) rc |= dalloc(&oi[q], d.n3());
-                if (rc) {
-                    for (double *&q : od) dfree(q);
-                    for (int32_t *&q : oi) dfree(q);
-                    return MGPU_ERR_NOMEM;
-                }
+            if (rc) {
+                for (double *&q : od) dfree(q);
+                for (int32_t *&q : oi) dfree(q);
+                return MGPU_ERR_NOMEM;
             }
-            for (int q = 0; q < 7; ++q) {
-                HIPCHK(hipMemcpyAsync(od[q], sd[q], b, kind, s));
-                vd[q] = od[q];
-            }
-            for (int q = 0; q < 6; ++q) {
-                HIPCHK(hipMemcpyAsync(oi[q], si[q], bi, kind, s));
-                vi[q] = oi[q];
-            }
+        }
+        CopySet c;
+        for (int q = 0; q < 7; ++q) {
+            vd[q] = view ? sd[q] : od[q];
+            if (!view && (q != 5 || want.visc) && (q != 6 || want.diffv)) c.add(sd[q], od[q], b);
+        }
+        for (int q = 0; q < 6; ++q) {
+            vi[q] = vmask ? si[q] : oi[q];
+            if (!vmask && want.masks) c.add(si[q], oi[q], bi);
+        }
+        if (a->device_pointers) {
+            if (int rc = launch_copy_set(c, s)) return rc;
+        } else {
+            for (int m = 0; m < c.n; ++m)
+                HIPCHK(hipMemcpyAsync(c.dst[m], c.src[m], (size_t)c.bytes[m], kind, s));
         }
         Qx = vd[0]; Qy = vd[1]; Qz = vd[2]; V = vd[3]; Vold = vd[4]; visc = vd[5]; diffv = vd[6];
         open = vi[0]; land = vi[1]; cfu = vi[2]; cfv = vi[3]; cfw = vi[4]; water = vi[5];
@@ -168,7 +182,7 @@ struct DevHydro {
         auto opt = [&](const auto *src, auto *&own, long n, auto *&at) -> int {
             // an array that the call itself writes is copied
             const void *v = src;
-            if (view && a->device_pointers && v != prop && v != a->PROPOld) {
+            if (view && v != prop && v != a->PROPOld) {
                 at = src;
                 return MGPU_SUCCESS;
             }
@@ -274,9 +288,10 @@ struct DevDerived {
     // hlines: also the list of implicit line rows (allocated on first use)
     // count: wait for the lists' lengths; without it (no other list than cols)
     // the column kernels read cols' length on the device
+    // cnt: with the wait, the four counters too
     int pack(const Dims &d, const DevHydro &h, const int32_t *kfloor, int docycle,
              hipStream_t s, bool tiles, bool hlines = false, const int32_t *dptr = nullptr,
-             bool count = true) {
+             bool count = true, unsigned long long *cnt = nullptr) {
         if (hlines && !hrows) {
             const long nw = (long)(d.wIUB - d.wILB + 1) * (d.wJUB - d.wJLB + 1) *
                             (d.wKUB - d.wKLB + 1);
@@ -300,6 +315,8 @@ struct DevDerived {
         }
         unsigned long long n[3];
         HIPCHK(hipMemcpyAsync(n, totals, sizeof(n), hipMemcpyDeviceToHost, s));
+        if (cnt)
+            HIPCHK(hipMemcpyAsync(cnt, counters, sizeof(*cnt) * 4, hipMemcpyDeviceToHost, s));
         HIPCHK(hipStreamSynchronize(s));
         ncells = cells ? (long)n[0] : 0;
         ncols = (long)n[1];
@@ -730,12 +747,18 @@ extern "C" int mgpu_ad_get_fluxes(mgpu_ad *ad, double *AdvFluxX, double *AdvFlux
     if (!ad) return MGPU_OFF_ERR;
     if (!ad->have_flux) return MGPU_ERR_STATE;      // GetAdvFlux ERR01 (AD:733)
     const size_t b3 = sizeof(double) * (size_t)ad->d.n3();
-    const hipMemcpyKind kind = device_pointers ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost;
     double *dst[6] = {AdvFluxX, AdvFluxY, AdvFluxZ, DifFluxX, DifFluxY, DifFluxZ};
     const double *src[6] = {ad->flux.afx, ad->flux.afy, ad->flux.afz,
                             ad->flux.dfx, ad->flux.dfy, ad->flux.dfz};
+    CopySet c;
     for (int q = 0; q < 6; ++q)
-        if (dst[q]) HIPCHK(hipMemcpyAsync(dst[q], src[q], b3, kind, ad->stream));
+        if (dst[q]) c.add(src[q], dst[q], b3);
+    if (device_pointers) {
+        if (int rc = launch_copy_set(c, ad->stream)) return rc;
+    } else {
+        for (int m = 0; m < c.n; ++m)
+            HIPCHK(hipMemcpyAsync(c.dst[m], c.src[m], b3, hipMemcpyDeviceToHost, ad->stream));
+    }
     HIPCHK(hipStreamSynchronize(ad->stream));
     return MGPU_SUCCESS;
 }
@@ -830,13 +853,38 @@ extern "C" int mgpu_ad_step(mgpu_ad *ad, const mgpu_ad_args *a, double *prop) {
         FluxArrays &q = ad->flux;
         HIPCHK(hipStreamSynchronize(s));
         if (dalloc(&q.afx, d.n3()) || dalloc(&q.afy, d.n3()) || dalloc(&q.afz, d.n3()) ||
-            dalloc(&q.dfx, d.n3()) || dalloc(&q.dfy, d.n3()) || dalloc(&q.dfz, d.n3()))
+            dalloc(&q.dfx, d.n3()) || dalloc(&q.dfy, d.n3()) || dalloc(&q.dfz, d.n3())) {
+            for (double **p : {&q.afx, &q.afy, &q.afz, &q.dfx, &q.dfy, &q.dfz}) dfree(*p);
             return MGPU_ERR_NOMEM;
+        }
+        // a call writes every WorkSize cell; the others stay zero
+        for (double *p : {q.afx, q.afy, q.afz, q.dfx, q.dfy, q.dfz})
+            HIPCHK(hipMemsetAsync(p, 0, b3, s));
     }
     const bool post = a->BoundaryCondition == 4 || a->BoundaryCondition == 8;
     if (post && (rc = ad->bnd.alloc(d))) return rc;
 
-    rc = ad->hydro.upload(d, a, s, true, prop);
+    // whether an earlier call's packed masks and lists serve this one
+    const void *src[8] = {a->OpenPoints3D, a->LandPoints3D, a->ComputeFacesU3D,
+                          a->ComputeFacesV3D, a->ComputeFacesW3D, a->WaterPoints3D,
+                          a->SmallDepths, (const void *)(intptr_t)a->device_pointers};
+    bool same = ad->masks_ok && !a->FirstProperty && a->DTProp == ad->mask_dt &&
+                ad->mask_disch == ad->disch.version && (sc.impH < 0 || ad->mask_hlines);
+    for (int q = 0; q < 8; ++q) same = same && src[q] == ad->mask_src[q];
+    // the conductances this call makes (see below)
+    const bool hfresh = !ad->have_faces || a->FirstProperty || a->DTProp != ad->last_dt ||
+                        a->schmidt_H != ad->last_schmidtH || a->NullDif;
+    const int do_h = sc.optimize ? first : hfresh;
+    const int do_v = sc.optimize ? first : 1;
+    DevHydro::Want want;
+    want.view = true;
+    // the raw masks are read by the packing, the open boundary and the passes
+    // after the solve alone; Visc_H and Diff_V by the conductances and the
+    // cell fluxes
+    want.masks = !same || a->ReferenceProp || post;
+    want.visc = do_h != 0;
+    want.diffv = do_v != 0 || cfl;
+    rc = ad->hydro.upload(d, a, s, want, prop);
     if (rc) return rc;
     double *P = ad->prop;
     if (a->device_pointers) P = prop;
@@ -850,24 +898,16 @@ extern "C" int mgpu_ad_step(mgpu_ad *ad, const mgpu_ad_args *a, double *prop) {
                                ad->disch.flow, s);
         if (rc) return rc;
     }
-    {
-        const void *src[8] = {a->OpenPoints3D, a->LandPoints3D, a->ComputeFacesU3D,
-                              a->ComputeFacesV3D, a->ComputeFacesW3D, a->WaterPoints3D,
-                              a->SmallDepths, (const void *)(intptr_t)a->device_pointers};
-        bool same = ad->masks_ok && !a->FirstProperty && a->DTProp == ad->mask_dt &&
-                    ad->mask_disch == ad->disch.version && (sc.impH < 0 || ad->mask_hlines);
-        for (int q = 0; q < 8; ++q) same = same && src[q] == ad->mask_src[q];
-        if (!same) {
-            ad->masks_ok = false;
-            rc = ad->der.pack(d, ad->hydro, ad->geom.KFloor, ad->docycle, s, false,
-                              sc.impH >= 0, ad->disch.on ? ad->disch.ptr : nullptr, false);
-            if (rc) return rc;
-            for (int q = 0; q < 8; ++q) ad->mask_src[q] = src[q];
-            ad->mask_dt = a->DTProp;
-            ad->mask_disch = ad->disch.version;
-            ad->mask_hlines = sc.impH >= 0;
-            ad->masks_ok = true;
-        }
+    if (!same) {
+        ad->masks_ok = false;
+        rc = ad->der.pack(d, ad->hydro, ad->geom.KFloor, ad->docycle, s, false, sc.impH >= 0,
+                          ad->disch.on ? ad->disch.ptr : nullptr, false);
+        if (rc) return rc;
+        for (int q = 0; q < 8; ++q) ad->mask_src[q] = src[q];
+        ad->mask_dt = a->DTProp;
+        ad->mask_disch = ad->disch.version;
+        ad->mask_hlines = sc.impH >= 0;
+        ad->masks_ok = true;
     }
     {
         // Convert_Visc_Dif_Horizontal(_opt) + Convert_Dif_Vertical (+ the
@@ -879,10 +919,6 @@ extern "C" int mgpu_ad_step(mgpu_ad *ad, const mgpu_ad_args *a, double *prop) {
         // keeps the U/V faces' while Set_Internal_State would (AD:5746-5835:
         // same model time -- a later property of the step --, same DTProp
         // and Schmidt number, no NullDif), NoDifFlux zeros included.
-        const bool hfresh = !ad->have_faces || a->FirstProperty || a->DTProp != ad->last_dt ||
-                            a->schmidt_H != ad->last_schmidtH || a->NullDif;
-        const int do_h = sc.optimize ? first : hfresh;
-        const int do_v = sc.optimize ? first : 1;
         const bool nf = !sc.optimize && a->NoDifFlux;
         rc = launch_prep_faces(d, ad->hydro.visc, ad->hydro.diffv, ad->hydro.Qx, ad->hydro.Qy,
                                ad->hydro.Qz, ad->geom.DUX, ad->geom.DVY, ad->geom.DZX,
@@ -1007,17 +1043,12 @@ extern "C" int mgpu_ad_step(mgpu_ad *ad, const mgpu_ad_args *a, double *prop) {
     // call reads it: at the ghost rows
     rc = launch_land_fill(d, ad->der.mask, ad->tig, tig0, s);
     if (!rc && sc.impH >= 0) rc = launch_copy_lines(d, sc.impH, ad->out, P, stop, s);
-    // the cell fluxes' explicit parts, with PROP before the solve (AD:1458-1468
-    // zero them first)
-    if (!rc && cfl) {
-        double *arr[6] = {ad->flux.afx, ad->flux.afy, ad->flux.afz,
-                          ad->flux.dfx, ad->flux.dfy, ad->flux.dfz};
-        for (double *q : arr) HIPCHK(hipMemsetAsync(q, 0, b3, s));
+    // the cell fluxes' explicit parts, with PROP before the solve
+    if (!rc && cfl)
         rc = launch_cell_flux_explicit(d, sc, f, P, ad->hydro.diffv, ad->geom.DZZ,
                                        a->SchmidtCoef_V, a->SchmidtBackground_V, a->NullDif,
                                        a->ImpExp_AdvV, a->ImpExp_DifV, ad->flux, ad->Rb,
                                        reinterpret_cast<unsigned int *>(ad->der.counters + 1), s);
-    }
     // Orlanski's exterior cells (written by the reference inside the open
     // boundary, before the solve; a solved cell among them takes the solve's
     // value, as there)
@@ -1347,6 +1378,7 @@ struct mgpu_transport {
     DevHydro hydro;
     DevDerived der;
     bool have_hydro = false;
+    bool masks_ok = false;   // the packed masks are those of the last set_hydro, which succeeded
     StepScalars sc;
     double schmidtH = 1.0, schmidtV = 1.0, backgroundV = 0.0;
     int nulldif = 0;
@@ -1524,6 +1556,7 @@ extern "C" int mgpu_transport_set_hydro(mgpu_transport *t, const mgpu_ad_args *a
         if (sc.vert && !t->mid && (rc = dalloc(&t->mid, ns))) return rc;
         if (!t->Rb && (rc = dalloc(&t->Rb, 4 * ns))) return rc;
     }
+    t->masks_ok = false;
     t->sc = sc;
     t->impdir = sc.impH;
     // WP:14576-14598 picks the optimised path for >= 2 TVD/SuperBee tracers
@@ -1531,26 +1564,27 @@ extern "C" int mgpu_transport_set_hydro(mgpu_transport *t, const mgpu_ad_args *a
     t->schmidtV = a->SchmidtCoef_V;
     t->backgroundV = a->SchmidtBackground_V;
     t->nulldif = a->NullDif;
-    rc = t->hydro.upload(t->d, a, t->stream);
+    DevHydro::Want want;
+    want.view_masks = true;
+    rc = t->hydro.upload(t->d, a, t->stream, want);
     if (rc) return rc;
     HIPCHK(hipMemsetAsync(t->der.counters, 0, t->der.counter_bytes, t->stream));
-    rc = t->der.pack(t->d, t->hydro, t->geom.KFloor, t->opts.docycle_method, t->stream,
-                     t->kernel == MGPU_KERNEL_SPLIT, sc.impH >= 0);
-    if (rc) return rc;
     unsigned long long cnt[4];
-    HIPCHK(hipMemcpyAsync(cnt, t->der.counters, sizeof(cnt), hipMemcpyDeviceToHost, t->stream));
-    HIPCHK(hipStreamSynchronize(t->stream));
+    rc = t->der.pack(t->d, t->hydro, t->geom.KFloor, t->opts.docycle_method, t->stream,
+                     t->kernel == MGPU_KERNEL_SPLIT, sc.impH >= 0, nullptr, true, cnt);
+    if (rc) return rc;
     if (cnt[2] & 0xffffffffu) return MGPU_ERR_MASKS;
     t->hydro_steps = 0;
     if ((rc = slot_sync(t))) return rc;
     // cells a step does not write (not solved under the new masks) keep their
     // latest value in both ping-pong buffers
-    HIPCHK(hipMemcpyAsync(t->buf[t->cur ^ 1], t->buf[t->cur],
-                          sizeof(double) * (size_t)t->d.n3() * (size_t)t->opts.ntracers,
-                          hipMemcpyDeviceToDevice, t->stream));
+    CopySet c;
+    c.add(t->buf[t->cur], t->buf[t->cur ^ 1],
+          sizeof(double) * (size_t)t->d.n3() * (size_t)t->opts.ntracers);
+    if ((rc = launch_copy_set(c, t->stream))) return rc;
     HIPCHK(hipStreamSynchronize(t->stream));
     drop_graphs(t);  // step scalars are baked into captured launches
-    t->have_hydro = true;
+    t->have_hydro = t->masks_ok = true;
     return MGPU_SUCCESS;
 }
 
@@ -1574,10 +1608,13 @@ extern "C" int mgpu_transport_set_tracer(mgpu_transport *t, int32_t index, const
                               hipMemcpyHostToDevice, t->stream));
         src = t->stage;
     }
-    // both ping-pong buffers start equal, so cells a step never writes
-    // (halos, land columns) stay identical in both
-    int rc = launch_interleave(n3, src, t->buf[0], t->opts.ntracers, index, 1, t->stream);
-    if (!rc) rc = launch_interleave(n3, src, t->buf[1], t->opts.ntracers, index, 1, t->stream);
+    // cells a step never writes (halos, land columns) are the same in both
+    // ping-pong buffers; the others a step writes before it reads them, once
+    // the masks are known (set_hydro copies the whole state again) and where
+    // no line solve leaves cells unwritten
+    const bool partial = t->masks_ok && t->impdir < 0 && t->kernel == MGPU_KERNEL_LANES;
+    int rc = launch_to_state(t->d, src, t->buf[t->cur], t->buf[t->cur ^ 1], t->opts.ntracers,
+                             index, partial ? t->der.mask : nullptr, t->stream);
     if (rc) return rc;
     HIPCHK(hipStreamSynchronize(t->stream));
     return MGPU_SUCCESS;
@@ -1589,7 +1626,7 @@ extern "C" int mgpu_transport_get_tracer(mgpu_transport *t, int32_t index, doubl
     if (!prop || index < 0 || index >= t->opts.ntracers) return MGPU_ERR_BADARG;
     const long n3 = t->d.n3();
     double *dst = dev ? prop : t->stage;
-    int rc = launch_interleave(n3, t->buf[t->cur], dst, t->opts.ntracers, index, 0, t->stream);
+    int rc = launch_from_state(n3, t->buf[t->cur], dst, t->opts.ntracers, index, t->stream);
     if (rc) return rc;
     if (!dev)
         HIPCHK(hipMemcpyAsync(prop, t->stage, sizeof(double) * (size_t)n3,

@@ -184,7 +184,8 @@ struct FluxArrays {
 };
 // The explicit parts (with PROP before the solve, P): the horizontal
 // advective and diffusive fluxes, and the vertical ones with weights
-// 1 - ImpExp_AdvV and 1 - ImpExp_DifV; the vertical advection coefficients
+// 1 - ImpExp_AdvV and 1 - ImpExp_DifV (zeros where a WorkSize face does not
+// compute); the vertical advection coefficients
 // of every W face go to coef (4 per cell) for the implicit part.
 int launch_cell_flux_explicit(const Dims &d, const StepScalars &sc, const SharedFields &f,
                               const double *P, const double *diffv, const double *DZZ,
@@ -374,10 +375,28 @@ int launch_transport(const TransportLaunch &L, const Dims &d, const StepScalars 
 // Whether launch_transport's column kernel is the depth-ordered walk, which
 // computes cw itself (the step's prep kernel may then skip cw).
 bool slot_walk(const TransportLaunch &L, const StepScalars &sc, const SharedFields &f);
-// Copy one tracer between a Fortran array (stride 1) and an interleaved
-// buffer (stride `stride`, slot t).  to_interleaved = 1: src Fortran -> dst.
-int launch_interleave(long n3, const double *src, double *dst, long stride, int t,
-                      int to_interleaved, hipStream_t s);
+// One tracer (a Fortran array) into slot t of the interleaved buffer cur, and
+// into other: everywhere (mask null), or where a step does not write.
+int launch_to_state(const Dims &d, const double *src, double *cur, double *other, long stride,
+                    int t, const uint8_t *mask, hipStream_t s);
+// Slot t of an interleaved buffer into a Fortran array.
+int launch_from_state(long n3, const double *src, double *dst, long stride, int t,
+                      hipStream_t s);
+// Device arrays copied by one launch (a launch each leaves the copies of
+// arrays of some tens of MB at 2.2 TB/s; together they reach the card's).
+// Lengths are multiples of 4 bytes.
+struct CopySet {
+    const void *src[16];
+    void *dst[16];
+    long bytes[16];
+    int n = 0;
+    void add(const void *a, void *b, size_t len) {
+        src[n] = a;
+        dst[n] = b;
+        bytes[n++] = (long)len;
+    }
+};
+int launch_copy_set(const CopySet &c, hipStream_t s);
 // Copies the cells of the implicit-advection lines (WorkSize lines along j
 // for axis 0, along i for axis 1, with their ghost end row) from src to dst,
 // unless *stop is non-zero.

@@ -197,15 +197,82 @@ int launch_slot_fields(const Dims &d, const SlotColumns &S, const double *Qz, co
 // ---------------------------------------------------------------------------
 // One tracer between a Fortran array and an interleaved buffer.
 namespace {
-__global__ void interleave_kernel(long n3, const double *__restrict__ src,
-                                  double *__restrict__ dst, long stride, int t, int to) {
+// A tracer into the state: every store of a wave touches a line per cell or
+// two, so a pass costs the whole state's lines whatever part of them it
+// writes.  Both ping-pong buffers take it in one pass, the second one (with
+// a mask) only at the cells no step writes: those outside the solved columns
+// and below WorkSize KLB.
+__global__ void to_state_kernel(Dims d, long n3, const double *__restrict__ src,
+                                double *__restrict__ cur, double *__restrict__ other, long stride,
+                                int t, const uint8_t *__restrict__ mask) {
+    const long top = (long)(d.wKUB - d.KLB) * d.sk;
     for (long x = blockIdx.x * (long)blockDim.x + threadIdx.x; x < n3;
          x += (long)gridDim.x * blockDim.x) {
-        if (to) dst[x * stride + t] = src[x];
-        else dst[x] = src[x * stride + t];
+        const double v = src[x];
+        cur[x * stride + t] = v;
+        bool keep = true;
+        if (mask) {
+            const uint32_t r = (uint32_t)((uint32_t)x % (uint32_t)d.sk);
+            const int j = d.JLB + (int)(r / (uint32_t)d.sj);
+            const int i = d.ILB + (int)(r % (uint32_t)d.sj);
+            const bool col = i >= d.wILB && i <= d.wIUB && j >= d.wJLB && j <= d.wJUB;
+            // the column solve writes rows KLB .. KUB + 1 of the WorkSize
+            keep = !(col && (uint32_t)x >= (uint32_t)d.sk && (mask[r + top] & M_WATER));
+        }
+        if (keep) other[x * stride + t] = v;
+    }
+}
+
+__global__ void from_state_kernel(long n3, const double *__restrict__ src,
+                                  double *__restrict__ dst, long stride, int t) {
+    for (long x = blockIdx.x * (long)blockDim.x + threadIdx.x; x < n3;
+         x += (long)gridDim.x * blockDim.x)
+        dst[x] = src[x * stride + t];
+}
+
+// The arrays of a set, one grid row each, 16 bytes a load where both ends
+// allow it, four loads in flight a lane.
+template <typename T>
+__device__ __forceinline__ void copy_units(const T *__restrict__ a, T *__restrict__ b, long n) {
+    const long nt = (long)gridDim.x * blockDim.x;
+    long q = blockIdx.x * (long)blockDim.x + threadIdx.x;
+    for (; q + 3 * nt < n; q += 4 * nt) {
+        const T v0 = a[q], v1 = a[q + nt], v2 = a[q + 2 * nt], v3 = a[q + 3 * nt];
+        b[q] = v0;
+        b[q + nt] = v1;
+        b[q + 2 * nt] = v2;
+        b[q + 3 * nt] = v3;
+    }
+    for (; q < n; q += nt) b[q] = a[q];
+}
+
+__global__ void __launch_bounds__(256) copy_set_kernel(CopySet c) {
+    const int m = blockIdx.y;
+    const char *a = static_cast<const char *>(c.src[m]);
+    char *b = static_cast<char *>(c.dst[m]);
+    const long n = c.bytes[m];
+    if ((((uintptr_t)a | (uintptr_t)b) & 15) == 0) {
+        copy_units(reinterpret_cast<const uint4 *>(a), reinterpret_cast<uint4 *>(b), n / 16);
+        if (blockIdx.x == 0 && threadIdx.x < (n % 16) / 4) {
+            const long q = n / 16 * 4 + threadIdx.x;
+            reinterpret_cast<uint32_t *>(b)[q] = reinterpret_cast<const uint32_t *>(a)[q];
+        }
+    } else {
+        copy_units(reinterpret_cast<const uint32_t *>(a), reinterpret_cast<uint32_t *>(b), n / 4);
     }
 }
 }  // namespace
+
+int launch_copy_set(const CopySet &c, hipStream_t s) {
+    if (c.n <= 0) return MGPU_SUCCESS;
+    long most = 0;
+    for (int m = 0; m < c.n; ++m) most = c.bytes[m] > most ? c.bytes[m] : most;
+    long blocks = (most / 64 + 255) / 256 + 1;
+    if (blocks > 2048) blocks = 2048;
+    hipLaunchKernelGGL(copy_set_kernel, dim3((unsigned)blocks, c.n), dim3(256), 0, s, c);
+    HIPCHK(hipGetLastError());
+    return MGPU_SUCCESS;
+}
 
 namespace {
 __global__ void disch_flow_kernel(int ncell, const int32_t *__restrict__ cbase,
@@ -561,22 +628,24 @@ __global__ void cell_flux_explicit_kernel(Dims d, StepScalars sc, SharedFields f
     const TracerSet ts{P, nullptr, 1, nullptr};
     int bad = 0;
     const bool hz = !sc.vertical1d;
+    // a face that does not compute has a zero flux (AD:1462-1468)
+    double afx = 0.0, afy = 0.0, afz = 0.0, dfx = 0.0, dfy = 0.0, dfz = 0.0;
     if (hz && (mk & M_CFU)) {
         // CalcHorizontalAdvFluxXX(_opt) (AD:3479-3567), weight 1 - ImpExp_AdvXX = 1
         double fl[1] = {0.0};
         if (!(f.xzero && f.xzero[x]))      // NoAdvFlux: cleared coefficients
             hface_flux<OPT, 1, false>(d, sc, f, ts, x, d.sj, j, d.JLB, d.JUB,
                                       f.DUX + d.idx2(i, j), d.sj, f.Qx[x], fl, bad);
-        o.afx[x] = 0.0 + 1.0 * fl[0];
+        afx = 0.0 + 1.0 * fl[0];
         // CalcHorizontalDifFluxXX(2) (AD:3784-3867)
-        o.dfx[x] = 0.0 - f.cu[x] * (P[x] - P[x - d.sj]);
+        dfx = 0.0 - f.cu[x] * (P[x] - P[x - d.sj]);
     }
     if (hz && !sc.xzflow && (mk & M_CFV)) {
         double fl[1];
         hface_flux<OPT, 1, false>(d, sc, f, ts, x, 1, i, d.ILB, d.IUB, f.DVY + d.idx2(i, j), 1,
                                   f.Qy[x], fl, bad);
-        o.afy[x] = 0.0 + 1.0 * fl[0];
-        o.dfy[x] = 0.0 - f.cv[x] * (P[x] - P[x - 1]);
+        afy = 0.0 + 1.0 * fl[0];
+        dfy = 0.0 - f.cv[x] * (P[x] - P[x - 1]);
     }
     if (sc.vert && (mk & M_CFW)) {
         // the W face's advection coefficients, from the stencil k-2 .. k+1
@@ -607,12 +676,18 @@ __global__ void cell_flux_explicit_kernel(Dims d, StepScalars sc, SharedFields f
                 const double pmm = (co[0].c == 0.0 || k - 2 < d.KLB) ? 0.0 : p[0][0];
                 fl = co[0].c * pmm + co[0].d * p[0][1] + co[0].e * p[0][2] + co[0].f * p[0][3];
             }
-            o.afz[x] = 0.0 + (1.0 - thA) * fl;
+            afz = 0.0 + (1.0 - thA) * fl;
         }
         if (thD < 1.0)
-            o.dfz[x] = 0.0 - vdif_term<OPT>(d, f, diffv, sV, bV, nulldif, DZZ, x, i, j, k,
-                                            1.0 - thD, P[x] - P[x - sk]);
+            dfz = 0.0 - vdif_term<OPT>(d, f, diffv, sV, bV, nulldif, DZZ, x, i, j, k, 1.0 - thD,
+                                       P[x] - P[x - sk]);
     }
+    o.afx[x] = afx;
+    o.afy[x] = afy;
+    o.afz[x] = afz;
+    o.dfx[x] = dfx;
+    o.dfy[x] = dfy;
+    o.dfz[x] = dfz;
     if (bad) atomicOr(badflag, 1u);
 }
 
@@ -764,12 +839,24 @@ int launch_land_fill(const Dims &d, const uint8_t *mask, double *dst, bool clear
     return MGPU_SUCCESS;
 }
 
-int launch_interleave(long n3, const double *src, double *dst, long stride, int t,
-                      int to_interleaved, hipStream_t s) {
+int launch_to_state(const Dims &d, const double *src, double *cur, double *other, long stride,
+                    int t, const uint8_t *mask, hipStream_t s) {
+    const long n3 = d.n3();
+    if (n3 >= (1L << 32)) mask = nullptr;   // the kernel's cell positions are 32-bit
     long blocks = (n3 + 255) / 256;
     if (blocks > 65536) blocks = 65536;
-    hipLaunchKernelGGL(interleave_kernel, dim3((unsigned)blocks), dim3(256), 0, s, n3, src, dst,
-                       stride, t, to_interleaved);
+    hipLaunchKernelGGL(to_state_kernel, dim3((unsigned)blocks), dim3(256), 0, s, d, n3, src, cur,
+                       other, stride, t, mask);
+    HIPCHK(hipGetLastError());
+    return MGPU_SUCCESS;
+}
+
+int launch_from_state(long n3, const double *src, double *dst, long stride, int t,
+                      hipStream_t s) {
+    long blocks = (n3 + 255) / 256;
+    if (blocks > 65536) blocks = 65536;
+    hipLaunchKernelGGL(from_state_kernel, dim3((unsigned)blocks), dim3(256), 0, s, n3, src, dst,
+                       stride, t);
     HIPCHK(hipGetLastError());
     return MGPU_SUCCESS;
 }

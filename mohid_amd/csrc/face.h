@@ -82,6 +82,13 @@ __device__ __forceinline__ double clamp_min_value(double dc) {
     return dc;
 }
 
+// clamp_min_value in three instructions; a NaN gives +-MIN_VALUE instead of
+// staying NaN (for a face whose flux has the NaN in it anyway).
+__device__ __forceinline__ double clamp_min_finite(double dc) {
+    dc = dc + 0.0;                                     // -0 counts as +0
+    return copysign(fmax(fabs(dc), MGPU_MIN_VALUE), dc);
+}
+
 // One instruction each for fmin and fmax; a NaN ratio gives 2 here as it does
 // with the reference's comparisons (only the sign of a zero may differ).
 __device__ __forceinline__ double superbee_theta(double r) {

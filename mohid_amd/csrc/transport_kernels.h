@@ -1446,12 +1446,22 @@ __device__ __forceinline__ void gather_line(const Dims &d, const SharedFields &f
     }
 }
 
-// hface_flux's optimised face over window o0 .. o0+3 of a gathered line;
-// with COEF its D and E coefficients go to fl and fe instead of the flux.
-template <int TPL, bool FAST, bool COEF = false>
-__device__ __forceinline__ void face_opt(const StepScalars &sc, const Line5<TPL> &L, int o0,
-                                         double Q, double (&fl)[TPL],
-                                         double (*fe)[TPL] = nullptr) {
+// hface_flux's optimised face over window o0 .. o0+3 of a gathered line.
+//
+// The kernels around it are bound by FP64 issue (72 % of the cycles at 8
+// tracers, 84 % in the fast mode at 4), so what the tracers share is made
+// once and the rest is short: with upstream value b, downstream value a and
+// h = (1 - Courant) / 2, theta = limiter * h (halving is exact, so this is the
+// reference's 0.5 * limiter * (1 - Courant)), h = 0 next to a closed cell, and
+// D p1 + E p2 is Q (1 - theta) b + Q theta a in either direction (a sum of two
+// commutes).
+//
+// Returns whether the face carries a flux (both its cells open); the flux in
+// fl is meant there.  With COEF its D and E coefficients go to fl and fe, zero
+// where it carries none.
+template <int TPL, bool FAST, bool COEF>
+__device__ __forceinline__ bool face_opt(const StepScalars &sc, const Line5<TPL> &L, int o0,
+                                         double Q, double (&fl)[TPL], double (&fe)[TPL]) {
     const bool o1 = o0 == 1;
     const double v1 = o1 ? L.v[2] : L.v[1], v2 = o1 ? L.v[3] : L.v[2];
     const double du0 = o1 ? L.du[1] : L.du[0], du1 = o1 ? L.du[2] : L.du[1];
@@ -1462,42 +1472,61 @@ __device__ __forceinline__ void face_opt(const StepScalars &sc, const Line5<TPL>
     const bool nearb = up ? !op0 : !op3;
     const double vup = up ? v1 : v2;
     const double cr = FAST ? Q * sc.dt * frcp(vup) : Q * sc.dt / vup;
+    const double h = nearb ? 0.0 : 0.5 * (1.0 - cr);
     const double s1 = du2 + du1;
     const double s0 = up ? du1 + du0 : du2 + du3;
-    const double i1 = FAST ? frcp(s1) : 0.0, i0 = FAST ? frcp(s0) : 0.0;
-    constexpr bool XR = !FAST && TPL >= 2;
-    const Recip R1 = XR ? recip(s1) : Recip{s1, 0.0, false};
-    const Recip R0 = XR ? recip(s0) : Recip{s0, 0.0, false};
     const bool act = op1 && op2;
+    double a[TPL], bb[TPL], dc[TPL], rr[TPL];
 #pragma unroll
     for (int t = 0; t < TPL; ++t) {
         const double q0 = o1 ? L.p[1][t] : L.p[0][t], q1 = o1 ? L.p[2][t] : L.p[1][t];
         const double q2 = o1 ? L.p[3][t] : L.p[2][t], q3 = o1 ? L.p[4][t] : L.p[3][t];
-        const double p1 = q1, p2 = q2;
+        a[t] = up ? q2 : q1;             // downstream, upstream
+        bb[t] = up ? q1 : q2;
+        dc[t] = a[t] - bb[t];
         // outside Size gather_line loaded q1 into q0 and q2 into q3
-        const double pf = up ? q0 : q3;
-        const double a = up ? p2 : p1, b = up ? p1 : p2;   // downstream, upstream
-        double dc, rr;
-        if (FAST) {
-            dc = clamp_min_value((a - b) * i1);
-            rr = (b - pf) * i0 * frcp(dc);
-        } else if (XR) {
-            dc = clamp_min_value(xdiv(a - b, R1));
-            rr = xdiv(b - pf, R0) / dc;
-        } else {
-            dc = clamp_min_value((a - b) / s1);
-            rr = (b - pf) / s0 / dc;
+        rr[t] = bb[t] - (up ? q0 : q3);
+    }
+    // the coefficients keep a NaN gradient; a flux has the NaN in it anyway
+    auto clamp = [](double v) { return COEF ? clamp_min_value(v) : clamp_min_finite(v); };
+    if constexpr (FAST) {
+        const double i1 = frcp(s1), i0 = frcp(s0);
+#pragma unroll
+        for (int t = 0; t < TPL; ++t) rr[t] = rr[t] * i0 * frcp(clamp(dc[t] * i1));
+    } else if constexpr (TPL == 1) {
+        rr[0] = rr[0] / s0 / clamp(dc[0] / s1);
+    } else {
+        // the shared spacings' reciprocals: the clamp and the limiter hide what
+        // fdiv's smallest quotients could differ in, so that only infinities and
+        // NaN need a test, one for the sum
+        const Recip R1 = recip(s1), R0 = recip(s0);
+        double qc[TPL], qr[TPL], sum = 0.0;
+#pragma unroll
+        for (int t = 0; t < TPL; ++t) {
+            qc[t] = fdiv(dc[t], R1);
+            qr[t] = fdiv(rr[t], R0);
+            sum = sum + fabs(qc[t]);
+            sum = sum + fabs(qr[t]);
         }
-        const double th = 0.5 * superbee_theta(rr) * (1.0 - cr);
-        const double Dc = nearb ? (up ? Q : 0.0) : (up ? Q * (1.0 - th) : Q * th);
-        const double Ec = nearb ? (up ? 0.0 : Q) : (up ? Q * th : Q * (1.0 - th));
+        if (!(R1.ok & R0.ok & (sum < 0x1p1000))) {
+#pragma unroll
+            for (int t = 0; t < TPL; ++t) { qc[t] = dc[t] / s1; qr[t] = rr[t] / s0; }
+        }
+#pragma unroll
+        for (int t = 0; t < TPL; ++t) rr[t] = qr[t] / clamp(qc[t]);
+    }
+#pragma unroll
+    for (int t = 0; t < TPL; ++t) {
+        const double th = superbee_theta(rr[t]) * h;
         if constexpr (COEF) {
-            fl[t] = act ? Dc : 0.0;
-            (*fe)[t] = act ? Ec : 0.0;
+            const double x = Q * (1.0 - th), y = Q * th;
+            fl[t] = act ? (up ? x : y) : 0.0;
+            fe[t] = act ? (up ? y : x) : 0.0;
         } else {
-            fl[t] = act ? Dc * p1 + Ec * p2 : 0.0;
+            fl[t] = Q * (1.0 - th) * bb[t] + Q * th * a[t];
         }
     }
+    return act;
 }
 
 // IMP >= 0: horizontal advection along j (0) or i (1) is implicit, and the
@@ -1522,72 +1551,94 @@ __device__ __forceinline__ void cell_rhs_opt(const Dims &d, const StepScalars &s
     // ---- then the arithmetic
     const double vk = LI.v[2];
     const bool open = mk & M_OPEN;
-    const double ivk = FAST ? frcp(vk) : 0.0;
-    const double dtv = dt * ivk;
-    const Recip Rv = FAST ? Recip{vk, 0.0, false} : recip(vk);
-    const double vv = open ? (FAST ? vold * ivk : xdiv(vold, Rv)) : 0.0;
     const bool hz = !sc.vertical1d;
     const bool cfu0 = hz && (mk & M_CFU);
     const bool cfu1 = hz && (mu1 & M_CFU);
     const bool cfv0 = hz && !sc.xzflow && (mk & M_CFV);
     const bool cfv1 = hz && !sc.xzflow && (mv1 & M_CFV);
-    const double au0 = cfu0 ? cu0 : 0.0, au1 = cfu1 ? cu1 : 0.0;
-    const double av0 = cfv0 ? cv0 : 0.0, av1 = cfv1 ? cv1 : 0.0;
-    const double wu0 = FAST ? au0 * dtv : 0.0, wu1 = FAST ? au1 * dtv : 0.0;
-    const double wv0 = FAST ? av0 * dtv : 0.0, wv1 = FAST ? av1 * dtv : 0.0;
-    const double bv0 = av0 * dt, bv1 = av1 * dt;
+    double pk[TPL];
+#pragma unroll
+    for (int t = 0; t < TPL; ++t) pk[t] = LI.p[2][t];
     // the advective face fluxes; for the implicit direction the faces' D
     // (fu*/fv*) and E (eu*/ev*) coefficients
     double fu0[TPL], fu1[TPL], fv0[TPL], fv1[TPL];
     double eu0[TPL], eu1[TPL], ev0[TPL], ev1[TPL];
-    face_opt<TPL, FAST, IMP == 0>(sc, LJ, 0, qu0, fu0, &eu0);
-    face_opt<TPL, FAST, IMP == 0>(sc, LJ, 1, qu1, fu1, &eu1);
-    face_opt<TPL, FAST, IMP == 1>(sc, LI, 0, qv0, fv0, &ev0);
-    face_opt<TPL, FAST, IMP == 1>(sc, LI, 1, qv1, fv1, &ev1);
-    // implicit rows: dt/V as the reference's DT1 = DT2 = DTProp / VolumeZ of
-    // the cell, and E0 of VolumeVariation
-    double dt2 = 0.0, E0 = 1.0;
+    const bool tu0 = face_opt<TPL, FAST, IMP == 0>(sc, LJ, 0, qu0, fu0, eu0);
+    const bool tu1 = face_opt<TPL, FAST, IMP == 0>(sc, LJ, 1, qu1, fu1, eu1);
+    const bool tv0 = face_opt<TPL, FAST, IMP == 1>(sc, LI, 0, qv0, fv0, ev0);
+    const bool tv1 = face_opt<TPL, FAST, IMP == 1>(sc, LI, 1, qv1, fv1, ev1);
+    // the faces whose flux enters TI (explicit directions)
+    const bool gu0 = IMP != 0 && cfu0 && tu0, gu1 = IMP != 0 && cfu1 && tu1;
+    const bool gv0 = IMP != 1 && cfv0 && tv0, gv1 = IMP != 1 && cfv1 && tv1;
+    // one face's terms of all tracers, where it computes
+    auto put = [&](bool on, double (&v)[TPL], auto term) {
+        if (on)
+#pragma unroll
+            for (int t = 0; t < TPL; ++t) v[t] = term(v[t], t);
+    };
+    double dt2 = 0.0;         // implicit rows: DTProp / VolumeZ of the cell
+    if constexpr (FAST) {
+        // the terms one by one, in the reference's order
+        const double dtv = dt * frcp(vk);
+        const double vv = open ? vold * frcp(vk) : 1.0;
+        const double wu0 = cu0 * dtv, wu1 = cu1 * dtv, wv0 = cv0 * dtv, wv1 = cv1 * dtv;
+#pragma unroll
+        for (int t = 0; t < TPL; ++t) {
+            double TI = pk[t] * vv;
+            disch_ti(f, x, open, pk[t], dt, vk, TI);
+            TIo[t] = TI;
+        }
+        put(cfu0, TIo, [&](double v, int t) { return v - wu0 * (pk[t] - LJ.p[1][t]); });
+        put(cfu1, TIo, [&](double v, int t) { return v + wu1 * (LJ.p[3][t] - pk[t]); });
+        put(cfv0, TIo, [&](double v, int t) { return v - wv0 * (pk[t] - LI.p[1][t]); });
+        put(cfv1, TIo, [&](double v, int t) { return v + wv1 * (LI.p[3][t] - pk[t]); });
+        put(gu0, TIo, [&](double v, int t) { return v + fu0[t] * dtv; });
+        put(gu1, TIo, [&](double v, int t) { return v - fu1[t] * dtv; });
+        put(gv0, TIo, [&](double v, int t) { return v + fv0[t] * dtv; });
+        put(gv1, TIo, [&](double v, int t) { return v - fv1[t] * dtv; });
+        dt2 = dtv;
+    } else {
+        // every quotient by V shares its reciprocal
+        const Recip Rv = recip(vk);
+        const double vv = open ? xdiv(vold, Rv) : 0.0;
+        const double bv0 = cv0 * dt, bv1 = cv1 * dt;
+        // the terms in the order the reference's loops deliver them
+        auto terms = [&](auto quot) {
+#pragma unroll
+            for (int t = 0; t < TPL; ++t) {
+                double TI = open ? pk[t] * vv : pk[t];
+                disch_ti(f, x, open, pk[t], dt, vk, TI);
+                TIo[t] = TI;
+            }
+            put(cfu0, TIo, [&](double v, int t) { return v - quot(cu0 * (pk[t] - LJ.p[1][t]) * dt); });
+            put(cfu1, TIo, [&](double v, int t) { return v + quot(cu1 * (LJ.p[3][t] - pk[t]) * dt); });
+            put(cfv0, TIo, [&](double v, int t) { return v - quot(bv0 * (pk[t] - LI.p[1][t])); });
+            put(cfv1, TIo, [&](double v, int t) { return v + quot(bv1 * (LI.p[3][t] - pk[t])); });
+            put(gu0, TIo, [&](double v, int t) { return v + quot(fu0[t] * dt); });
+            put(gu1, TIo, [&](double v, int t) { return v - quot(fu1[t] * dt); });
+            put(gv0, TIo, [&](double v, int t) { return v + quot(fv0[t] * dt); });
+            put(gv1, TIo, [&](double v, int t) { return v - quot(fv1[t] * dt); });
+        };
+        terms([&](double n) { return fdiv(n, Rv); });
+        // fdiv's bits are the division's for every term a sum of this size can
+        // show: one test of the sums instead of one per term
+        bool ok = Rv.ok;
+#pragma unroll
+        for (int t = 0; t < TPL; ++t) {
+            const double m = fabs(TIo[t]);
+            ok = ok & (m < 0x1p1000) & ((m >= 0x1p-300) | (m == 0.0));
+        }
+        if (!ok) terms([&](double n) { return n / vk; });
+        if (IMP >= 0) dt2 = xdiv(dt, Rv);
+    }
     if constexpr (IMP >= 0) {
-        dt2 = FAST ? dt * frcp(vk) : xdiv(dt, Rv);
+        // dt/V as the reference's DT1 = DT2, and E0 of VolumeVariation
+        double E0 = 1.0;
         if (k == d.wKUB && open) E0 = 1.0 + dt2 * qz1;
         disch_e(f, x, open, dt, vk, E0);
-    }
-    const bool au = IMP != 0, av = IMP != 1;   // explicit directions
+        const bool c0 = IMP == 0 ? cfu0 : cfv0, c1 = IMP == 0 ? cfu1 : cfv1;
 #pragma unroll
-    for (int t = 0; t < TPL; ++t) {
-        const double pk = LI.p[2][t];
-        double TI = open ? pk * vv : pk;
-        disch_ti(f, x, open, pk, dt, vk, TI);
-        if (cfu0) {
-            const double g = pk - LJ.p[1][t];
-            TI = FAST ? TI - wu0 * g : TI - xdiv(au0 * g * dt, Rv);
-        }
-        if (cfu1) {
-            const double g = LJ.p[3][t] - pk;
-            TI = FAST ? TI + wu1 * g : TI + xdiv(au1 * g * dt, Rv);
-        }
-        if (cfv0) {
-            const double g = pk - LI.p[1][t];
-            TI = FAST ? TI - wv0 * g : TI - xdiv(bv0 * g, Rv);
-        }
-        if (cfv1) {
-            const double g = LI.p[3][t] - pk;
-            TI = FAST ? TI + wv1 * g : TI + xdiv(bv1 * g, Rv);
-        }
-        if (FAST) {
-            if (au && cfu0) TI = TI + fu0[t] * dtv;
-            if (au && cfu1) TI = TI - fu1[t] * dtv;
-            if (av && cfv0) TI = TI + fv0[t] * dtv;
-            if (av && cfv1) TI = TI - fv1[t] * dtv;
-        } else {
-            if (au && cfu0) TI = TI + xdiv(fu0[t] * dt, Rv);
-            if (au && cfu1) TI = TI - xdiv(fu1[t] * dt, Rv);
-            if (av && cfv0) TI = TI + xdiv(fv0[t] * dt, Rv);
-            if (av && cfv1) TI = TI - xdiv(fv1[t] * dt, Rv);
-        }
-        TIo[t] = TI;
-        if constexpr (IMP >= 0) {
-            const bool c0 = IMP == 0 ? cfu0 : cfv0, c1 = IMP == 0 ? cfu1 : cfv1;
+        for (int t = 0; t < TPL; ++t) {
             const double d0 = IMP == 0 ? fu0[t] : fv0[t], e0 = IMP == 0 ? eu0[t] : ev0[t];
             const double d1 = IMP == 0 ? fu1[t] : fv1[t], e1 = IMP == 0 ? eu1[t] : ev1[t];
             double E = E0;
@@ -1625,7 +1676,7 @@ explicit_lane_kernel(Dims d, StepScalars sc, SharedFields f, TracerSet ts,
                      const uint32_t *__restrict__ cells, long ncells, double *__restrict__ TW,
                      SlotColumns S, unsigned int *__restrict__ badflag) {
     constexpr int LPC = NT / TPL;   // lanes per cell
-    const long g = xcd_tile(blockIdx.x, gridDim.x) * 256 + threadIdx.x;
+    const long g = xcd_tile32(blockIdx.x, gridDim.x) * 256 + threadIdx.x;
     const long n = g / LPC;
     if (n >= ncells) return;
     const int t0 = (int)(g - n * LPC) * TPL;
@@ -3309,7 +3360,10 @@ static int launch_explicit_lanes(int want, const Dims &d, const StepScalars &sc,
     if constexpr (NT == 1) return launch_explicit_tiles<OPT, FAST>(d, sc, f, ts, l, TW, bad, s);
     else {
     if (!l.cells) return MGPU_ERR_STATE;
-    switch (lane_tpl<NT>(want, 4)) {
+    // 2 in FP64 (1024 x 1024 x 40, 8 tracers: 1.96 ms, 2.23 with 4 and 2.77 with
+    // 1), 4 in the fast mode, which needs fewer registers (60 levels, 4 tracers:
+    // 2.10 ms, 2.96 with 2)
+    switch (lane_tpl<NT>(want, FAST ? 4 : 2)) {
         case 8: if constexpr (NT % 8 == 0) return launch_explicit_tpl<OPT, NT, 8, FAST>(d, sc, f, ts, l, TW, bad, s); break;
         case 4: if constexpr (NT % 4 == 0) return launch_explicit_tpl<OPT, NT, 4, FAST>(d, sc, f, ts, l, TW, bad, s); break;
         case 2: if constexpr (NT % 2 == 0) return launch_explicit_tpl<OPT, NT, 2, FAST>(d, sc, f, ts, l, TW, bad, s); break;

@@ -94,6 +94,37 @@ def test_columns_vertical_schemes(impV, difV, optimize):
     _check(case, case.tracers, optimize)
 
 
+@pytest.mark.parametrize("tracers", (2, 4, 8))
+def test_batched_zero_and_small_values(tracers):
+    """Launches of several tracers: a patch in exact zeros, at 1 and at 1e-200,
+    and the values beside it, in one launch."""
+    from mohid_amd.advection_diffusion import Transport
+    case = fx.make_case(fx.config("c3", ni=70, nj=19, nk=5, kfloor=(1, 5), land_frac=0.3,
+                                  tracers=("lognormal",) * tracers, **GRID))
+    wet = case.hydro["WaterPoints3D"] == 1
+    props = []
+    for t in range(tracers):
+        p = np.array(case.tracers[t], order="F", copy=True)
+        far = np.zeros_like(wet)
+        far[30:] = True
+        if t % 2 == 0:
+            p[wet & far] = 0.0
+        if t % 4 == 0:
+            p[wet & ~far] *= 1e-200
+        props.append(p)
+    tr = Transport(case.size, case.worksize, case.geom, tracers)
+    tr.set_hydro(case.hydro, case.params)
+    for t, p in enumerate(props):
+        tr.set_tracer(t, p)
+    tr.run(3)
+    ref = ora.run_case(case, 3, nthreads=1, tracers=props)
+    solved = np.zeros(props[0].shape, dtype=bool)
+    solved[:, :, 1:] = (case.hydro["WaterPoints3D"][:, :, case.worksize[5]] == 1)[:, :, None]
+    for t in range(tracers):
+        assert np.array_equal(tr.get_tracer(t)[solved], ref[t][solved]), t
+    tr.close()
+
+
 @pytest.mark.parametrize("tracers,order", [(3, 0), (3, 1), (5, 0), (5, 1)])
 def test_batched_columns(tracers, order):
     """Interleaved tracers, columns in memory order and by first row."""

@@ -1370,10 +1370,6 @@ struct mgpu_transport {
     Dims d;
     mgpu_transport_opts opts;
     hipStream_t stream = nullptr;
-    // second stream for the next step's face conductances, forked from and
-    // joined back into `stream` by the two events
-    hipStream_t side = nullptr;
-    hipEvent_t fork = nullptr, join = nullptr;
     DevGeometry geom;
     DevHydro hydro;
     DevDerived der;
@@ -1442,12 +1438,8 @@ static void drop_graphs(mgpu_transport *t) {
 extern "C" int mgpu_transport_destroy(mgpu_transport *t) {
     if (!t) return MGPU_OFF_ERR;
     if (t->stream) (void)hipStreamSynchronize(t->stream);
-    if (t->side) (void)hipStreamSynchronize(t->side);
     drop_graphs(t);
     drop_events(t);
-    if (t->fork) (void)hipEventDestroy(t->fork);
-    if (t->join) (void)hipEventDestroy(t->join);
-    if (t->side) (void)hipStreamDestroy(t->side);
     t->geom.release();
     t->hydro.release();
     t->der.release();
@@ -1504,13 +1496,6 @@ extern "C" int mgpu_transport_create(const mgpu_size3d *size, const mgpu_size3d 
     if (e != hipSuccess) {
         mgpu_set_error("hipStreamCreate", e);
         delete t;
-        return MGPU_ERR_HIP;
-    }
-    if ((e = hipStreamCreate(&t->side)) != hipSuccess ||
-        (e = hipEventCreateWithFlags(&t->fork, hipEventDisableTiming)) != hipSuccess ||
-        (e = hipEventCreateWithFlags(&t->join, hipEventDisableTiming)) != hipSuccess) {
-        mgpu_set_error("side stream", e);
-        mgpu_transport_destroy(t);
         return MGPU_ERR_HIP;
     }
     const long n3 = t->d.n3();
@@ -1735,7 +1720,6 @@ static int enqueue_steps(mgpu_transport *t, int nsteps, int cur, int dir) {
                                  nf ? t->hydro.nfw : nullptr, 1, sw ? 0 : 1, t->der.cu,
                                  t->der.cv, t->der.cw, q);
     };
-    bool ahead = false;   // this step's conductances were enqueued on the side stream
     for (int st = 0; st < nsteps; ++st) {
         StepScalars sc = t->sc;
         if (dir >= 0) {
@@ -1762,34 +1746,20 @@ static int enqueue_steps(mgpu_transport *t, int nsteps, int cur, int dir) {
         L.counters = t->der.counters;
         L.mid = t->mid;
         L.Rb = t->Rb;
-        const bool sw = slot_walk(L, sc, f);
-        // The depth-ordered walk reads no conductance, so the next step's
-        // (the same inputs, the same operations) are made on the side stream
-        // while this step's walk runs, after this step's first kernels have
-        // read cu and cv; the next step's first kernels wait for them.
-        // Per-kernel timing keeps every kernel on the handle's stream.
-        const bool overlap = sw && !t->timing && st + 1 < nsteps;
+        // The conductances depend on nothing a step changes (the hydrodynamic
+        // state stays for the whole run): the run's first step makes them for
+        // all.  (Made again every step, on a second stream beside the column
+        // walk, they cost 0.25 ms of 4.3 a step at 1024 x 1024 x 40 with 8
+        // tracers and 0.5 of 5.2 in the fast mode at 60 levels.)
         int rc;
-        if (ahead) {
-            HIPCHK(hipStreamWaitEvent(s, t->join, 0));
-        } else {
-            if ((rc = mark(t))) return rc;
-            if ((rc = prep(sw, s))) return rc;
-            if ((rc = mark(t))) return rc;
-        }
-        ahead = false;
+        if ((rc = mark(t))) return rc;
+        if (st == 0 && (rc = prep(slot_walk(L, sc, f), s))) return rc;
+        if ((rc = mark(t))) return rc;
         // first kernel(s) of every chunk, then the second kernel(s)
         for (int ph = 1; ph <= 2; ++ph) {
             rc = launch_transport(L, d, sc, f, s, ph);
             if (rc) return rc;
             if ((rc = mark(t))) return rc;
-            if (ph == 1 && overlap) {
-                HIPCHK(hipEventRecord(t->fork, s));
-                HIPCHK(hipStreamWaitEvent(t->side, t->fork, 0));
-                if ((rc = prep(sw, t->side))) return rc;
-                HIPCHK(hipEventRecord(t->join, t->side));
-                ahead = true;
-            }
         }
         cur ^= 1;
     }

@@ -75,6 +75,9 @@ struct StepScalars {
     // 3-D implicit horizontal advection: the vertical step restarts from the
     // identity rows with TI = PROP after the line solves (AD:4245-4248)
     int hreset;
+    // whether the column walk writes the inert rows' null_real (a batched run's
+    // third step and later ones find it in both state buffers)
+    int nulls = 1;
 };
 
 // Discharges of a drop-in call (SetDischarges, AD:978-1034), one entry per

@@ -2092,7 +2092,8 @@ column_lane_kernel(Dims d, StepScalars sc, SharedFields f, TracerSet ts,
         double nr[TPL];
 #pragma unroll
         for (int u = 0; u < TPL; ++u) nr[u] = MGPU_NULL_REAL;
-        for (int k = d.wKLB; k < ks && k <= KUB; ++k) store_tpl<TPL>(t1.out + (base + k * sk) * s, nr);
+        for (int k = d.wKLB; sc.nulls && k < ks && k <= KUB; ++k)
+            store_tpl<TPL>(t1.out + (base + k * sk) * s, nr);
     }
     if (bad) atomicOr(badflag, 1u);
 }
@@ -2378,7 +2379,8 @@ column_pipe_kernel(Dims d, StepScalars sc, SharedFields f, TracerSet ts,
         double nr[TPL];
 #pragma unroll
         for (int u = 0; u < TPL; ++u) nr[u] = MGPU_NULL_REAL;
-        for (int k = d.wKLB; k < ks && k <= KUB; ++k) store_tpl<TPL>(t1.out + (base + k * sk) * s, nr);
+        for (int k = d.wKLB; sc.nulls && k < ks && k <= KUB; ++k)
+            store_tpl<TPL>(t1.out + (base + k * sk) * s, nr);
     }
     if (bad) atomicOr(badflag, 1u);
 }
@@ -2597,7 +2599,7 @@ column_quad_kernel(Dims d, StepScalars sc, SharedFields f, TracerSet ts,
     }
     // the inert land rows below the column's first row (AD:1753), stored last,
     // so that out may be P itself
-    if (act)
+    if (act && sc.nulls)
         for (int k = d.wKLB + l; k < ks && k <= KUB; k += 4)
             t1.out[(base + k * sk) * s] = MGPU_NULL_REAL;
     if (bad) atomicOr(badflag, 1u);
@@ -3204,7 +3206,8 @@ slot_map_kernel(const uint32_t *__restrict__ cols, long nc, int32_t *__restrict_
 }  // namespace
 
 // Lane-variant launches with TPL tracers per lane (1, 2, 4 or 8 dividing NT;
-// 0 picks the default: 4 in the explicit kernel, 2 in the column walk).
+// 0 picks the default: 2 (4 in the fast mode) in the explicit kernel, 1 or 2 in
+// the column walk).
 // One tracer: tiles, with every face computed once.
 template <bool OPT, bool FAST>
 static int launch_explicit_tiles(const Dims &d, const StepScalars &sc, const SharedFields &f,
@@ -3380,7 +3383,13 @@ static int launch_column_lanes(int want, const Dims &d, const StepScalars &sc,
                                unsigned int *bad, hipStream_t s, int mixed = 0,
                                bool walk = false) {
     if (walk && want > 4) want = 4;
-    switch (lane_tpl<NT>(want, 2)) {
+    // one tracer a lane keeps 17 levels of W and G on chip, two keep 8 but need
+    // half the lanes: one while the columns have 28 rows or fewer on average
+    // (KFloor 5..40 at 1024 x 1024, 8 tracers: walk 1.63 ms, 1.86 with two), two
+    // for deeper ones (700 x 700, 40 full levels, 5 steps of 8 tracers: 15.6
+    // ms, 16.2 with one)
+    const bool shallow = l.ncells > 0 && l.ncells <= 28 * l.ncols;
+    switch (lane_tpl<NT>(want, shallow ? 1 : 2)) {
         case 8: if constexpr (NT % 8 == 0) return launch_column_tpl<OPT, NT, 8, FAST>(d, sc, f, ts, l, TW, Gs, counters, bad, s, mixed, walk); break;
         case 4: if constexpr (NT % 4 == 0) return launch_column_tpl<OPT, NT, 4, FAST>(d, sc, f, ts, l, TW, Gs, counters, bad, s, mixed, walk); break;
         case 2: if constexpr (NT % 2 == 0) return launch_column_tpl<OPT, NT, 2, FAST>(d, sc, f, ts, l, TW, Gs, counters, bad, s, mixed, walk); break;

@@ -14,8 +14,8 @@ int launch_pack_masks(const Dims &d, const int32_t *open, const int32_t *land,
                       const int32_t *kfloor, int docycle, uint8_t *mask, int32_t *kstart,
                       uint32_t *colcnt, unsigned int *flags, hipStream_t s) {
     const int nI = d.IUB - d.ILB + 1, nJ = d.JUB - d.JLB + 1;
-    hipLaunchKernelGGL(mask_columns_kernel, dim3((nI + 63) / 64, nJ), dim3(64, 4), 0, s, d, open,
-                       land, cfu, cfv, cfw, water, small, dptr, kfloor, docycle, mask, kstart,
+    hipLaunchKernelGGL(mask_columns_kernel, dim3((unsigned)((nI + 63) / 64) * (unsigned)nJ),
+                       dim3(64, 4), 0, s, d, open, land, cfu, cfv, cfw, water, small, dptr, kfloor, docycle, mask, kstart,
                        colcnt, flags);
     HIPCHK(hipGetLastError());
     return MGPU_SUCCESS;

@@ -55,7 +55,8 @@ namespace {
 // rows above.  kstart is the first row above the inert bottom rows.
 //
 // One pass over the six int32 masks (bound by their 24 bytes a cell): a block
-// takes 64 columns of one j, its four waves a quarter of the levels each, and
+// takes 64 columns of one j (blocks along i, then j, in one grid dimension: the
+// others end at 65,535), its four waves a quarter of the levels each, and
 // makes the mask bytes, kstart, the checks of the masks and the count of the
 // row's solved columns.  At 512 x 512 x 50 the pass took 104 us, and kstart
 // from the bytes another 23; together now 108.
@@ -68,7 +69,8 @@ mask_columns_kernel(Dims d, const int32_t *__restrict__ open, const int32_t *__r
                     uint8_t *__restrict__ mask, int32_t *__restrict__ kstart,
                     uint32_t *__restrict__ colcnt, unsigned int *__restrict__ flags) {
     __shared__ int first[4][64];
-    const int i = d.ILB + (int)(blockIdx.x * 64 + threadIdx.x), j = d.JLB + (int)blockIdx.y;
+    const unsigned nib = (unsigned)((d.IUB - d.ILB + 64) / 64), jj = blockIdx.x / nib;
+    const int i = d.ILB + (int)((blockIdx.x - jj * nib) * 64 + threadIdx.x), j = d.JLB + (int)jj;
     const int part = threadIdx.y;
     const bool in = i <= d.IUB;
     const bool col = in && i >= d.wILB && i <= d.wIUB && j >= d.wJLB && j <= d.wJUB;

@@ -35,7 +35,8 @@ def _check(case, props, optimize):
 @pytest.mark.parametrize("optimize", (False, True))
 @pytest.mark.parametrize("ni,nj,nk,kfloor,land", [
     (3, 3, 1, (1, 1), 0.0), (63, 7, 3, (1, 3), 0.2), (64, 8, 2, (1, 1), 0.0),
-    (65, 9, 4, (2, 4), 0.4), (129, 17, 5, (1, 5), 0.3), (2, 40, 6, (1, 6), 0.1)])
+    (65, 9, 4, (2, 4), 0.4), (129, 17, 5, (1, 5), 0.3), (2, 40, 6, (1, 6), 0.1),
+    (2, 70000, 2, (1, 2), 0.0), (70000, 2, 2, (1, 2), 0.0)])
 def test_extents(ni, nj, nk, kfloor, land, optimize):
     case = fx.make_case(fx.config("c3", ni=ni, nj=nj, nk=nk, kfloor=kfloor, land_frac=land,
                                   tracers=("temperature", "lognormal"), **GRID))

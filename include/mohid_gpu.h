@@ -288,7 +288,10 @@ typedef struct {
 int mgpu_transport_create(const mgpu_size3d *size, const mgpu_size3d *worksize,
                           const mgpu_transport_opts *opts, const mgpu_geometry *geometry,
                           mgpu_transport **out);
-/* Shared per-step inputs (the arrays of mgpu_ad_args; scalars from args). */
+/* Shared per-step inputs (the arrays of mgpu_ad_args; scalars from args).  After
+ * a call that fails once it has begun to take them over (MGPU_ERR_MASKS, a HIP
+ * error) mgpu_transport_run returns MGPU_ERR_STATE until a call succeeds; the
+ * tracers stay as they were. */
 int mgpu_transport_set_hydro(mgpu_transport *t, const mgpu_ad_args *args);
 /* The geometry of the following steps, as mgpu_ad_set_geometry (the
  * reference's per-call GetGeometryDistances / GetGeometryAreas, AD:1353-1401,

@@ -1541,7 +1541,11 @@ extern "C" int mgpu_transport_set_hydro(mgpu_transport *t, const mgpu_ad_args *a
         if (sc.vert && !t->mid && (rc = dalloc(&t->mid, ns))) return rc;
         if (!t->Rb && (rc = dalloc(&t->Rb, 4 * ns))) return rc;
     }
-    t->masks_ok = false;
+    // From here on the handle's masks, fields and scalars are replaced: a call
+    // that fails part-way leaves a mixture of two states, and tracers set after
+    // the last one that succeeded are whole in one state buffer only
+    // (mgpu_transport_set_tracer).  mgpu_transport_run refuses until a call succeeds.
+    t->masks_ok = t->have_hydro = false;
     t->sc = sc;
     t->impdir = sc.impH;
     // WP:14576-14598 picks the optimised path for >= 2 TVD/SuperBee tracers

@@ -1,6 +1,7 @@
 """Tracers and fields into and out of a batched handle (GPU): tracers set again
-between runs reach both state buffers, and device arrays at any 8-byte (fields)
-or 4-byte (masks) alignment give the same step, equal to the oracle."""
+between runs reach both state buffers, no step runs after refused masks, and
+device arrays at any 8-byte (fields) or 4-byte (masks) alignment give the same
+step, equal to the oracle."""
 import numpy as np
 import pytest
 
@@ -35,6 +36,44 @@ def test_tracers_set_between_runs(steps):
         tr.set_tracer(t, p)
     tr.run(steps)
     ref = ora.run_case(case, steps, nthreads=1, tracers=props)
+    for t in range(len(names)):
+        assert np.array_equal(tr.get_tracer(t), ref[t]), t
+    tr.close()
+
+
+@pytest.mark.parametrize("use_graph", (False, True))
+def test_masks_refused_between_runs(use_graph):
+    """No step runs after a hydrodynamic state whose masks were refused, not even
+    one captured before it; the tracers set meanwhile are whole once the next
+    state is accepted."""
+    from mohid_amd import _lib as L
+    from mohid_amd.advection_diffusion import Transport
+    names = ("temperature", "salinity", "lognormal")
+    case = _case(names)
+    tr = Transport(case.size, case.worksize, case.geom, len(names))
+    tr.set_hydro(case.hydro, case.params)
+    for t, p in enumerate(case.tracers):
+        tr.set_tracer(t, p)
+    tr.run(1, use_graph=use_graph)
+    rng = np.random.default_rng(5)
+    props = [np.asfortranarray(p + rng.uniform(0, 1, p.shape)) for p in case.tracers]
+    for t, p in enumerate(props):
+        tr.set_tracer(t, p)
+    # a W face missing above the floor of a column: not what KFloor says
+    cfw = np.array(case.hydro["ComputeFacesW3D"], order="F", copy=True)
+    i, j, k = np.argwhere(cfw[:, :, :case.worksize[5]] == 1)[0]   # below the surface one
+    cfw[i, j, k] = 0
+    with pytest.raises(L.MgpuError) as e:
+        tr.set_hydro(dict(case.hydro, ComputeFacesW3D=cfw), case.params)
+    assert e.value.code == L.MGPU_ERR_MASKS
+    with pytest.raises(L.MgpuError) as e:
+        tr.run(1, use_graph=use_graph)
+    assert e.value.code == L.MGPU_ERR_STATE
+    for t, p in enumerate(props):
+        assert np.array_equal(tr.get_tracer(t), p), t
+    tr.set_hydro(case.hydro, case.params)
+    tr.run(2, use_graph=use_graph)
+    ref = ora.run_case(case, 2, nthreads=1, tracers=props)
     for t in range(len(names)):
         assert np.array_equal(tr.get_tracer(t), ref[t]), t
     tr.close()

@@ -1756,6 +1756,7 @@ __device__ __forceinline__ void tile_face(const Dims &d, const StepScalars &sc,
         // Q (1 - theta) b + Q theta a in either (a sum of two commutes), and
         // the first-order flux next to a closed cell has theta = 0.
         double th = 0.0;
+        bool stops = false;
         if (OPT || sc.methodH == TVD) {
             const double vup = up ? v1 : v2;
             const double cr = FAST && OPT ? Q * sc.dt * frcp(vup) : Q * sc.dt / vup;
@@ -1770,15 +1771,18 @@ __device__ __forceinline__ void tile_face(const Dims &d, const StepScalars &sc,
                 const double dc = clamp_min_value((a - bb) / s1);
                 rr = (bb - pf) / s0 / dc;
             }
-            const double l = OPT ? superbee_theta(rr) : limiter_theta(sc.tvdH, rr, bad);
+            int unknown = 0;
+            const double l = OPT ? superbee_theta(rr) : limiter_theta(sc.tvdH, rr, unknown);
             th = nearb ? 0.0 : 0.5 * l * (1.0 - cr);
+            // the limiter counts only where the face uses it
+            stops = nearb ? !OPT && !sc.up2H : unknown != 0;
         }
         x = Q * (1.0 - th) * bb + Q * th * a;
         if (!OPT) {
             // the reference's zero C and F coefficients
             const double z = Q * 0.0;
             x = x + z * (in0 ? x0 : 0.0) + z * p3;
-            if (sc.methodH == TVD && nearb && !sc.up2H) {   // the reference stops here
+            if (stops) {                         // the reference stops here
                 x = 0.0;
                 if (op1 && op2) bad = 1;
             }

@@ -54,6 +54,26 @@ def test_faces(method, limiter, up2):
     _check(case, case.tracers, False)
 
 
+@pytest.mark.parametrize("ni,closed", [(2, ()), (3, (3,))])
+def test_limiter_that_no_face_uses(ni, closed):
+    """A limiter id that does not exist matters only where a face takes its value:
+    not beside a closed cell with Upwind2H, nor at a face with a closed cell."""
+    from mohid_amd import _lib as L
+    from mohid_amd.advection_diffusion import AdvectionDiffusion
+    case = fx.make_case(fx.config("c2", ni=ni, nj=2, nk=4, depth=(8.0, 20.0), **GRID))
+    for i in closed:
+        case.hydro["OpenPoints3D"][i] = 0
+    case.params.update(TVDLimitationH=99, Upwind2H=True)
+    _check(case, case.tracers, False)
+    # where one does, the call says so
+    case.params["Upwind2H"] = False
+    gpu = AdvectionDiffusion(case.size, case.worksize, case.geom)
+    with pytest.raises(L.MgpuError) as e:
+        gpu(np.array(case.tracers[0], order="F", copy=True), case.hydro, case.params)
+    assert e.value.code == L.MGPU_ERR_OPTION
+    gpu.kill()
+
+
 @pytest.mark.parametrize("optimize", (False, True))
 def test_zero_and_small_values(optimize):
     """Exact zeros beside a patch, and the patch at 1e-200: every quotient is

@@ -84,10 +84,15 @@ struct DevGeometry {
             return MGPU_ERR_BADARG;
         const size_t b2 = sizeof(double) * (size_t)d.n2(), b3 = sizeof(double) * (size_t)d.n3();
         CopySet c;
-        c.add(g->DUX, DUX, b2); c.add(g->DVY, DVY, b2); c.add(g->DZX, DZX, b2);
-        c.add(g->DZY, DZY, b2); c.add(g->KFloorZ, KFloor, sizeof(int32_t) * (size_t)d.n2());
-        c.add(g->AreaU, AreaU, b3); c.add(g->AreaV, AreaV, b3); c.add(g->DZZ, DZZ, b3);
-        c.add(g->DWZ, DWZ, b3);
+        const struct {
+            const void *from;
+            void *to;
+            size_t len;
+        } all[] = {{g->DUX, DUX, b2}, {g->DVY, DVY, b2}, {g->DZX, DZX, b2}, {g->DZY, DZY, b2},
+                   {g->KFloorZ, KFloor, sizeof(int32_t) * (size_t)d.n2()},
+                   {g->AreaU, AreaU, b3}, {g->AreaV, AreaV, b3}, {g->DZZ, DZZ, b3},
+                   {g->DWZ, DWZ, b3}};
+        for (const auto &q : all) c.add(q.from, q.to, q.len, q.from);
         if (g->device_pointers) {
             if (int rc = launch_copy_set(c, s)) return rc;
         } else {
@@ -138,7 +143,7 @@ struct DevHydro {
     int upload(const Dims &d, const mgpu_ad_args *a, hipStream_t s, Want want,
                const double *prop = nullptr) {
         const bool view = want.view && a->device_pointers;
-        const bool vmask = (want.view || want.view_masks) && a->device_pointers;
+        bool vmask = (want.view || want.view_masks) && a->device_pointers;
         const hipMemcpyKind kind =
             a->device_pointers ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
         const size_t b = sizeof(double) * (size_t)d.n3(), bi = sizeof(int32_t) * (size_t)d.n3();
@@ -146,6 +151,9 @@ struct DevHydro {
                                a->Visc_H, a->Diff_V};
         const int32_t *si[6] = {a->OpenPoints3D, a->LandPoints3D, a->ComputeFacesU3D,
                                 a->ComputeFacesV3D, a->ComputeFacesW3D, a->WaterPoints3D};
+        // what the batched transport copies, and the optional arrays of a drop-in
+        // call, may lie on another device: viewed only where kernels reach them
+        for (int q = 0; q < 6 && vmask && !view; ++q) vmask = on_device(si[q], s);
         const double *vd[7];
         const int32_t *vi[6];
         if ((!view && !od[6]) || (!vmask && !oi[5])) {
@@ -164,11 +172,12 @@ struct DevHydro {
         CopySet c;
         for (int q = 0; q < 7; ++q) {
             vd[q] = view ? sd[q] : od[q];
-            if (!view && (q != 5 || want.visc) && (q != 6 || want.diffv)) c.add(sd[q], od[q], b);
+            if (!view && (q != 5 || want.visc) && (q != 6 || want.diffv))
+                c.add(sd[q], od[q], b, sd[q]);
         }
         for (int q = 0; q < 6; ++q) {
             vi[q] = vmask ? si[q] : oi[q];
-            if (!vmask && want.masks) c.add(si[q], oi[q], bi);
+            if (!vmask && want.masks) c.add(si[q], oi[q], bi, si[q]);
         }
         if (a->device_pointers) {
             if (int rc = launch_copy_set(c, s)) return rc;
@@ -182,7 +191,7 @@ struct DevHydro {
         auto opt = [&](const auto *src, auto *&own, long n, auto *&at) -> int {
             // an array that the call itself writes is copied
             const void *v = src;
-            if (view && v != prop && v != a->PROPOld) {
+            if (view && v != prop && v != a->PROPOld && on_device(v, s)) {
                 at = src;
                 return MGPU_SUCCESS;
             }
@@ -752,7 +761,7 @@ extern "C" int mgpu_ad_get_fluxes(mgpu_ad *ad, double *AdvFluxX, double *AdvFlux
                             ad->flux.dfx, ad->flux.dfy, ad->flux.dfz};
     CopySet c;
     for (int q = 0; q < 6; ++q)
-        if (dst[q]) c.add(src[q], dst[q], b3);
+        if (dst[q]) c.add(src[q], dst[q], b3, dst[q]);
     if (device_pointers) {
         if (int rc = launch_copy_set(c, ad->stream)) return rc;
     } else {
@@ -1569,7 +1578,7 @@ extern "C" int mgpu_transport_set_hydro(mgpu_transport *t, const mgpu_ad_args *a
     // latest value in both ping-pong buffers
     CopySet c;
     c.add(t->buf[t->cur], t->buf[t->cur ^ 1],
-          sizeof(double) * (size_t)t->d.n3() * (size_t)t->opts.ntracers);
+          sizeof(double) * (size_t)t->d.n3() * (size_t)t->opts.ntracers, nullptr);
     if ((rc = launch_copy_set(c, t->stream))) return rc;
     HIPCHK(hipStreamSynchronize(t->stream));
     drop_graphs(t);  // step scalars are baked into captured launches

@@ -83,7 +83,10 @@ __device__ __forceinline__ double clamp_min_value(double dc) {
 }
 
 // clamp_min_value in three instructions; a NaN gives +-MIN_VALUE instead of
-// staying NaN (for a face whose flux has the NaN in it anyway).
+// staying NaN.  Only where the sum that takes the face's flux is NaN then anyway:
+// a face's gradient is NaN for a length that is NaN, two lengths of 0 between equal
+// values, or infinite values on both sides, and the diffusive term of the same
+// face, made of the same lengths (prep_faces_kernel) and values, is NaN with it.
 __device__ __forceinline__ double clamp_min_finite(double dc) {
     dc = dc + 0.0;                                     // -0 counts as +0
     return copysign(fmax(fabs(dc), MGPU_MIN_VALUE), dc);

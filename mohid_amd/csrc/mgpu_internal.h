@@ -385,17 +385,23 @@ int launch_to_state(const Dims &d, const double *src, double *cur, double *other
 // Slot t of an interleaved buffer into a Fortran array.
 int launch_from_state(long n3, const double *src, double *dst, long stride, int t,
                       hipStream_t s);
+// Whether p is memory of stream s's own device: what its kernels may read and
+// write in place.
+bool on_device(const void *p, hipStream_t s);
 // Device arrays copied by one launch (a launch each leaves the copies of
-// arrays of some tens of MB at 2.2 TB/s; together they reach the card's).
-// Lengths are multiples of 4 bytes.
+// arrays of some tens of MB at 2.2 TB/s; together they reach the card's);
+// arrays that lie elsewhere than on the stream's device are copied by the
+// runtime.  Lengths are multiples of 4 bytes.
 struct CopySet {
     const void *src[16];
     void *dst[16];
     long bytes[16];
+    const void *caller[16];   // the end that is the caller's (null: both are the handle's)
     int n = 0;
-    void add(const void *a, void *b, size_t len) {
+    void add(const void *a, void *b, size_t len, const void *callers) {
         src[n] = a;
         dst[n] = b;
+        caller[n] = callers;
         bytes[n++] = (long)len;
     }
 };

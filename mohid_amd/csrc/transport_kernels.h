@@ -1489,7 +1489,7 @@ __device__ __forceinline__ bool face_opt(const StepScalars &sc, const Line5<TPL>
         // outside Size gather_line loaded q1 into q0 and q2 into q3
         rr[t] = bb[t] - (up ? q0 : q3);
     }
-    // the coefficients keep a NaN gradient; a flux has the NaN in it anyway
+    // the coefficients keep a NaN gradient; a flux needs not (clamp_min_finite)
     auto clamp = [](double v) { return COEF ? clamp_min_value(v) : clamp_min_finite(v); };
     if constexpr (FAST) {
         const double i1 = frcp(s1), i0 = frcp(s0);

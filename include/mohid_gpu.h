@@ -279,7 +279,8 @@ typedef struct {
     int32_t kernel;                       /* MGPU_KERNEL_AUTO / _FUSED / _SPLIT / _LANES */
     int32_t tracers_per_launch;           /* 1..8 tracers per kernel launch; 0: 8 */
     int32_t explicit_tracers_per_lane;    /* lanes: 1, 2, 4 or 8 (dividing the launch); 0: 2, FAST 4 */
-    int32_t column_tracers_per_lane;      /* lanes: 1, 2, 4 or 8 (dividing the launch); 0: 1 or 2 by depth */
+    int32_t column_tracers_per_lane;      /* lanes: 1, 2, 4 or 8 (dividing the launch); 0: 1 or 2 by depth;
+                                             of the lane walk (see MGPU_WALK_AUTO) */
     int32_t refinements;                  /* MGPU_PREC_MIXED: residual-and-correction passes of
                                              the column solve per step, 1..4 (0: 2); the first
                                              starts from the tracer before the step */
@@ -338,6 +339,18 @@ int mgpu_transport_set_kernel(mgpu_transport *t, int32_t kernel);
 #define MGPU_COLUMNS_AUTO 2
 #define MGPU_SLOT_MIN_STEPS 4
 int mgpu_transport_set_column_order(mgpu_transport *t, int32_t order);
+/* Form of the FP64/FAST column walk of the lane variant and of a drop-in
+ * handle.  MGPU_WALK_LANES: one lane takes a column for one or several tracers
+ * (column_tracers_per_lane).  MGPU_WALK_QUADS: four lanes share a column of one
+ * tracer, whatever column_tracers_per_lane says, where its forward sweep fits
+ * LDS (255 levels; deeper columns take the lane walk).  MGPU_WALK_AUTO (the
+ * default): quads for few columns, lanes for many.  Results do not depend on
+ * it.  No counterpart in the reference. */
+#define MGPU_WALK_AUTO 0
+#define MGPU_WALK_LANES 1
+#define MGPU_WALK_QUADS 2
+int mgpu_transport_set_column_walk(mgpu_transport *t, int32_t walk);
+int mgpu_ad_set_column_walk(mgpu_ad *ad, int32_t walk);
 int mgpu_transport_destroy(mgpu_transport *t);
 /* Waits for the handle's work; MGPU_ERR_OPTION if a face method or limiter
  * the reference stops on was met since the last set_hydro, MGPU_ERR_PIVOT

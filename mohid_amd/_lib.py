@@ -38,6 +38,9 @@ MGPU_COLUMNS_MEMORY = 0
 MGPU_COLUMNS_BY_DEPTH = 1
 MGPU_COLUMNS_AUTO = 2
 MGPU_SLOT_MIN_STEPS = 4
+MGPU_WALK_AUTO = 0
+MGPU_WALK_LANES = 1
+MGPU_WALK_QUADS = 2
 MGPU_NOALLOC_MAX_CELLS = 16777216
 
 STATUS_NAMES = {
@@ -102,6 +105,7 @@ EXPORTS = (
     "mgpu_transport_set_tracer",
     "mgpu_transport_get_tracer", "mgpu_transport_run", "mgpu_transport_tracer_ptr",
     "mgpu_transport_set_lanes", "mgpu_transport_set_kernel", "mgpu_transport_set_column_order",
+    "mgpu_transport_set_column_walk", "mgpu_ad_set_column_walk",
     "mgpu_transport_stream", "mgpu_transport_destroy", "mgpu_transport_timing",
     "mgpu_transport_kernel_times",
     "mgpu_selfcheck_xdiv", "mgpu_version", "mgpu_last_error",
@@ -162,6 +166,8 @@ def lib():
     L.mgpu_transport_set_lanes.argtypes = [vp, ct.c_int32, ct.c_int32, ct.c_int32]
     L.mgpu_transport_set_kernel.argtypes = [vp, ct.c_int32]
     L.mgpu_transport_set_column_order.argtypes = [vp, ct.c_int32]
+    L.mgpu_transport_set_column_walk.argtypes = [vp, ct.c_int32]
+    L.mgpu_ad_set_column_walk.argtypes = [vp, ct.c_int32]
     L.mgpu_transport_destroy.argtypes = [vp]
     L.mgpu_transport_timing.argtypes = [vp, ct.c_int32, ct.c_int32]
     L.mgpu_transport_kernel_times.argtypes = [vp, ct.POINTER(ct.c_double),

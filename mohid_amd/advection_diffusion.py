@@ -173,6 +173,11 @@ class AdvectionDiffusion:
         g = _geometry(geometry, keep)
         L.check("mgpu_ad_set_geometry", L.lib().mgpu_ad_set_geometry(self._h, ct.byref(g)))
 
+    def set_column_walk(self, walk: int) -> None:
+        """Form of the column walk (MGPU_WALK_LANES, _QUADS or _AUTO, the
+        default); results do not depend on it."""
+        L.check("mgpu_ad_set_column_walk", L.lib().mgpu_ad_set_column_walk(self._h, int(walk)))
+
     def set_discharges(self, d: Dict) -> None:
         """SetDischarges (AD:978-1034) from a dict of arrays: per discharge
         cell flow, conc, concMF, I, J, K, Kmin, Kmax; per discharge vert,
@@ -358,6 +363,12 @@ class Transport:
         L.check("mgpu_transport_set_column_order",
                 L.lib().mgpu_transport_set_column_order(self._h, int(order)))
         self.column_order = int(order)
+
+    def set_column_walk(self, walk: int) -> None:
+        """Form of the FP64/FAST column walk (MGPU_WALK_LANES, _QUADS or _AUTO,
+        the default); results do not depend on it."""
+        L.check("mgpu_transport_set_column_walk",
+                L.lib().mgpu_transport_set_column_walk(self._h, int(walk)))
 
     def stream_handle(self) -> int:
         s = ct.c_void_p()

@@ -528,6 +528,7 @@ struct mgpu_ad {
     double last_dt = 0.0, last_schmidtH = 0.0;   // Set_Internal_State's memory (AD:5746)
     unsigned long long last_zero_pivots = 0;
     unsigned long long *cnt = nullptr;      // pinned: the counters of a call
+    int walk = MGPU_WALK_AUTO;              // form of the column walk
 };
 
 extern "C" int mgpu_ad_create(const mgpu_size3d *size, const mgpu_size3d *worksize,
@@ -1030,6 +1031,7 @@ extern "C" int mgpu_ad_step(mgpu_ad *ad, const mgpu_ad_args *a, double *prop) {
     L.counters = ad->der.counters;
     L.tig = tig0 ? nullptr : ad->tig;
     L.Rb = ad->Rb;
+    L.lanes.walk = ad->walk;
     const unsigned long long *stop = ad->der.counters + 3;
     if (sc.hreset) {
         // line solves into mid (a copy of PROP, so that it is PROP after
@@ -1411,6 +1413,7 @@ struct mgpu_transport {
     // first row (SlotStore), in memory order, or by first row once the
     // current hydrodynamic state has run MGPU_SLOT_MIN_STEPS steps
     int col_order = MGPU_COLUMNS_AUTO;
+    int walk = MGPU_WALK_AUTO;   // form of the FP64/FAST column walk
     long hydro_steps = 0;   // steps run since the last set_hydro
     SlotStore slot;
 };
@@ -1707,6 +1710,27 @@ extern "C" int mgpu_transport_set_column_order(mgpu_transport *t, int32_t order)
     return t->have_hydro ? slot_sync(t) : MGPU_SUCCESS;
 }
 
+static bool walk_ok(int32_t w) {
+    return w == MGPU_WALK_AUTO || w == MGPU_WALK_LANES || w == MGPU_WALK_QUADS;
+}
+
+extern "C" int mgpu_transport_set_column_walk(mgpu_transport *t, int32_t walk) {
+    if (!t) return MGPU_OFF_ERR;
+    if (!walk_ok(walk)) return MGPU_ERR_BADARG;
+    if (walk == t->walk) return MGPU_SUCCESS;
+    HIPCHK(hipStreamSynchronize(t->stream));
+    t->walk = walk;
+    drop_graphs(t);   // captured launches bake the walk in
+    return MGPU_SUCCESS;
+}
+
+extern "C" int mgpu_ad_set_column_walk(mgpu_ad *ad, int32_t walk) {
+    if (!ad) return MGPU_OFF_ERR;
+    if (!walk_ok(walk)) return MGPU_ERR_BADARG;
+    ad->walk = walk;
+    return MGPU_SUCCESS;
+}
+
 extern "C" int mgpu_transport_stream(mgpu_transport *t, void **stream) {
     if (!t) return MGPU_OFF_ERR;
     if (!stream) return MGPU_ERR_BADARG;
@@ -1760,6 +1784,7 @@ static int enqueue_steps(mgpu_transport *t, int nsteps, int cur, int dir) {
         L.lists.slot = t->slot.view(t->schmidtV, t->backgroundV);
         L.lanes.explicit_tpl = t->opts.explicit_tracers_per_lane;
         L.lanes.column_tpl = t->opts.column_tracers_per_lane;
+        L.lanes.walk = t->walk;
         L.counters = t->der.counters;
         L.mid = t->mid;
         L.Rb = t->Rb;

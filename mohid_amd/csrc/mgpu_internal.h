@@ -302,6 +302,7 @@ int launch_slot_fields(const Dims &d, const SlotColumns &S, const double *Qz, co
 // Tracers per lane of the lane variant's kernels (0: library default).
 struct LaneShape {
     int explicit_tpl = 0, column_tpl = 0;
+    int walk = MGPU_WALK_AUTO;   // form of the FP64/FAST column walk
     // MGPU_PREC_MIXED: FP64 residual-and-correction passes of the column
     // solve (column_mixed_kernel); 0: the FP64 (or FAST) column kernel
     int mixed = 0;

@@ -3253,19 +3253,23 @@ static inline long quad_lds(const Dims &d) {
 // ragged columns, 28,000 / 44,000 / 63,000 lines of 40 levels 62 -> 42,
 // 65 -> 59, 79 -> 83 us; other path, 40 full levels, 40,000 / 90,000 / 122,000
 // lines 132 -> 65, 167 -> 125, 176 -> 185 us.
+// form: MGPU_WALK_LANES keeps the lane walk, MGPU_WALK_QUADS the quad walk
+// wherever a column fits.
 template <bool OPT>
-static inline bool quad_columns(const Dims &d, long lines) {
-    return lines <= (OPT ? 48L : 96L) * 1024 && quad_lds(d) <= 65536;
+static inline bool quad_columns(const Dims &d, long lines, int form) {
+    return quad_lds(d) <= 65536 &&
+           (form == MGPU_WALK_QUADS ||
+            (form == MGPU_WALK_AUTO && lines <= (OPT ? 48L : 96L) * 1024));
 }
 
 template <bool OPT, int NT, int TPL, bool FAST>
 static int launch_column_tpl(const Dims &d, const StepScalars &sc, const SharedFields &f,
                              const TracerSet &ts, const SolveLists &l, double *TW, double *Gs,
                              unsigned long long *counters, unsigned int *bad, hipStream_t s,
-                             int mixed = 0, bool walk = false) {
+                             int mixed, bool walk, int form) {
     const long nb = (l.ncols * (NT / TPL) + 255) / 256;
     if (nb <= 0) return MGPU_SUCCESS;
-    if (!walk && mixed <= 0 && quad_columns<OPT>(d, l.ncols * NT)) {
+    if (!walk && mixed <= 0 && quad_columns<OPT>(d, l.ncols * NT, form)) {
         const bool slot = OPT && !f.obc.bp && !f.disch.ptr && l.slot.cols;
         if (slot && l.slot.ncols != l.ncols) return MGPU_ERR_STATE;
         const unsigned nq = (unsigned)((l.ncols * NT + 15) / 16);
@@ -3383,11 +3387,12 @@ static int launch_explicit_lanes(int want, const Dims &d, const StepScalars &sc,
 }
 
 template <bool OPT, int NT, bool FAST>
-static int launch_column_lanes(int want, const Dims &d, const StepScalars &sc,
+static int launch_column_lanes(const LaneShape &lanes, const Dims &d, const StepScalars &sc,
                                const SharedFields &f, const TracerSet &ts, const SolveLists &l,
                                double *TW, double *Gs, unsigned long long *counters,
                                unsigned int *bad, hipStream_t s, int mixed = 0,
                                bool walk = false) {
+    int want = lanes.column_tpl;
     if (walk && want > 4) want = 4;
     // one tracer a lane keeps 17 levels of W and G on chip, two keep 8 but need
     // half the lanes: one while the columns have 28 rows or fewer on average
@@ -3396,13 +3401,13 @@ static int launch_column_lanes(int want, const Dims &d, const StepScalars &sc,
     // ms, 16.2 with one)
     const bool shallow = l.ncells > 0 && l.ncells <= 28 * l.ncols;
     switch (lane_tpl<NT>(want, shallow ? 1 : 2)) {
-        case 8: if constexpr (NT % 8 == 0) return launch_column_tpl<OPT, NT, 8, FAST>(d, sc, f, ts, l, TW, Gs, counters, bad, s, mixed, walk); break;
-        case 4: if constexpr (NT % 4 == 0) return launch_column_tpl<OPT, NT, 4, FAST>(d, sc, f, ts, l, TW, Gs, counters, bad, s, mixed, walk); break;
-        case 2: if constexpr (NT % 2 == 0) return launch_column_tpl<OPT, NT, 2, FAST>(d, sc, f, ts, l, TW, Gs, counters, bad, s, mixed, walk); break;
+        case 8: if constexpr (NT % 8 == 0) return launch_column_tpl<OPT, NT, 8, FAST>(d, sc, f, ts, l, TW, Gs, counters, bad, s, mixed, walk, lanes.walk); break;
+        case 4: if constexpr (NT % 4 == 0) return launch_column_tpl<OPT, NT, 4, FAST>(d, sc, f, ts, l, TW, Gs, counters, bad, s, mixed, walk, lanes.walk); break;
+        case 2: if constexpr (NT % 2 == 0) return launch_column_tpl<OPT, NT, 2, FAST>(d, sc, f, ts, l, TW, Gs, counters, bad, s, mixed, walk, lanes.walk); break;
         default: break;
     }
     return launch_column_tpl<OPT, NT, 1, FAST>(d, sc, f, ts, l, TW, Gs, counters, bad, s, mixed,
-                                               walk);
+                                               walk, lanes.walk);
 }
 
 template <bool OPT, int NT, int TPL, bool FAST>
@@ -3471,7 +3476,7 @@ static int launch_chunk(int variant, int phase, const Dims &d, const StepScalars
         }
         if ((phase & 2) && sc.vert) {
             const TracerSet tc{imp.mid, ts.out, ts.s, imp.tig ? imp.tig : imp.mid};
-            const int rc = launch_column_lanes<OPT, NT, FAST>(lanes.column_tpl, d, sc, f, tc,
+            const int rc = launch_column_lanes<OPT, NT, FAST>(lanes, d, sc, f, tc,
                                                               lists, Wb, Gb, counters, bad, s);
             if (rc) return rc;
         }
@@ -3484,7 +3489,7 @@ static int launch_chunk(int variant, int phase, const Dims &d, const StepScalars
             if (rc) return rc;
         }
         if (phase & 2) {
-            const int rc = launch_column_lanes<OPT, NT, FAST>(lanes.column_tpl, d, sc, f, ts,
+            const int rc = launch_column_lanes<OPT, NT, FAST>(lanes, d, sc, f, ts,
                                                               lists, Wb, Gb, counters, bad, s,
                                                               lanes.mixed);
             if (rc) return rc;
@@ -3495,7 +3500,7 @@ static int launch_chunk(int variant, int phase, const Dims &d, const StepScalars
         // one walk per column: the explicit right-hand side inside it
         if (lanes.mixed) return MGPU_ERR_UNSUPPORTED;
         if (phase & 1) {
-            const int rc = launch_column_lanes<OPT, NT, FAST>(lanes.column_tpl, d, sc, f, ts,
+            const int rc = launch_column_lanes<OPT, NT, FAST>(lanes, d, sc, f, ts,
                                                               lists, Wb, Gb, counters, bad, s, 0,
                                                               true);
             if (rc) return rc;

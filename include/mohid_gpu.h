@@ -279,8 +279,9 @@ typedef struct {
     int32_t kernel;                       /* MGPU_KERNEL_AUTO / _FUSED / _SPLIT / _LANES */
     int32_t tracers_per_launch;           /* 1..8 tracers per kernel launch; 0: 8 */
     int32_t explicit_tracers_per_lane;    /* lanes: 1, 2, 4 or 8 (dividing the launch); 0: 2, FAST 4 */
-    int32_t column_tracers_per_lane;      /* lanes: 1, 2, 4 or 8 (dividing the launch); 0: 1 or 2 by depth;
-                                             of the lane walk (see MGPU_WALK_AUTO) */
+    int32_t column_tracers_per_lane;      /* lanes: 1, 2, 4 or 8 (dividing the launch); 0: by the kernel,
+                                             the lines and the columns' depths.  Of the lane
+                                             walk (see MGPU_WALK_AUTO) */
     int32_t refinements;                  /* MGPU_PREC_MIXED: residual-and-correction passes of
                                              the column solve per step, 1..4 (0: 2); the first
                                              starts from the tracer before the step */

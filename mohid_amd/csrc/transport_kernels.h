@@ -3212,8 +3212,8 @@ slot_map_kernel(const uint32_t *__restrict__ cols, long nc, int32_t *__restrict_
 }  // namespace
 
 // Lane-variant launches with TPL tracers per lane (1, 2, 4 or 8 dividing NT;
-// 0 picks the default: 2 (4 in the fast mode) in the explicit kernel, 1 or 2 in
-// the column walk).
+// 0 picks the default: 2 (4 in the fast mode) in the explicit kernel,
+// column_default in the column solve).
 // One tracer: tiles, with every face computed once.
 template <bool OPT, bool FAST>
 static int launch_explicit_tiles(const Dims &d, const StepScalars &sc, const SharedFields &f,
@@ -3386,6 +3386,46 @@ static int launch_explicit_lanes(int want, const Dims &d, const StepScalars &sc,
     }
 }
 
+// Tracers a lane of the column solve where none are set.  More tracers a lane
+// share the row's loads and arithmetic, fewer leave more lanes and (in the
+// pipelined walk) keep more levels of W and G on chip, so the better number
+// depends on the kernel, the lines (columns x tracers) and how ragged the columns
+// are.  Measured in us of the kernel, FP64 unless said, 25 % land, one / two (/
+// four) tracers a lane:
+//   up to three waves a SIMD, one in every kernel but the fused walk: pipelined
+//     walk, 187k lines of 40 levels 121 / 146, of 10 31 / 34; other path 170 /
+//     187; MIXED (86k, 24 levels) 127 / 136 / 188.  From 280k on they are equal or
+//     two is better (other path, 327k: 184 / 142);
+//   other path (column_lane_kernel), two: 500 x 500 x 40, T = 4 560 / 472, ragged
+//     505 / 443;
+//   MIXED, four: 500 x 500 x 40, T = 8 2,380 / 2,161 / 1,725, ragged 1,971 / 1,850 /
+//     1,492;
+//   fused walk, one or four by lines: T = 4, 330 x 330 410 / 466 / 473, 1024 x 1024
+//     3,484 / 3,700 / 2,888 (24 levels); FAST two: 3,144 / 2,118 / 2,470;
+//   pipelined walk, full columns, two: 1024 x 1024, T = 8, 10 levels 731 / 570, 40
+//     levels 3,210 / 2,850, T = 4 1,667 / 1,610.  (60 levels of T = 4 in the fast
+//     mode by depth prefer one at 1024 x 1024, 2,375 / 2,505, and two at 500 x
+//     500, 608 / 593: two there as well.)
+//   pipelined walk, ragged columns (KFloor up to 40, mean rows 20 to 32), one for up
+//     to four tracers (T = 4 1,596 / 1,735 by depth, 1,367 / 1,447 in memory order)
+//     and, by depth, for more (T = 8 1,563 / 1,720; memory order 2,309 / 2,258)
+//     unless the columns are shallow (20 levels, mean 11 rows: 805 / 755).  Where
+//     the mean is 37 of 40 rows two is better again (2,720 / 2,370 by depth), where
+//     it is 32 one (2,660 / 3,080): the line is at 34.
+template <int NT, bool FAST>
+static int column_default(const Dims &d, const SolveLists &l, bool pipe, bool mixed, bool walk) {
+    constexpr long WAVES = 65536;             // lanes of a wave on every SIMD
+    const long lines = l.ncols * NT;
+    if (walk) return FAST ? 2 : (NT % 4 == 0 && lines > 6 * WAVES ? 4 : 1);
+    if (lines <= 3 * WAVES) return 1;
+    if (mixed) return 4;
+    if (!pipe) return 2;
+    const long nk = d.wKUB - d.wKLB + 1;
+    const bool ragged = 20 * l.ncells <= 17 * l.ncols * nk;
+    const bool by_depth = l.slot.cols != nullptr;
+    return ragged && (NT <= 4 || (by_depth && l.ncells > 14 * l.ncols)) ? 1 : 2;
+}
+
 template <bool OPT, int NT, bool FAST>
 static int launch_column_lanes(const LaneShape &lanes, const Dims &d, const StepScalars &sc,
                                const SharedFields &f, const TracerSet &ts, const SolveLists &l,
@@ -3394,13 +3434,8 @@ static int launch_column_lanes(const LaneShape &lanes, const Dims &d, const Step
                                bool walk = false) {
     int want = lanes.column_tpl;
     if (walk && want > 4) want = 4;
-    // one tracer a lane keeps 17 levels of W and G on chip, two keep 8 but need
-    // half the lanes: one while the columns have 28 rows or fewer on average
-    // (KFloor 5..40 at 1024 x 1024, 8 tracers: walk 1.63 ms, 1.86 with two), two
-    // for deeper ones (700 x 700, 40 full levels, 5 steps of 8 tracers: 15.6
-    // ms, 16.2 with one)
-    const bool shallow = l.ncells > 0 && l.ncells <= 28 * l.ncols;
-    switch (lane_tpl<NT>(want, shallow ? 1 : 2)) {
+    const bool pipe = OPT && mixed <= 0 && !walk && !f.obc.bp && !f.disch.ptr;
+    switch (lane_tpl<NT>(want, column_default<NT, FAST>(d, l, pipe, mixed > 0, walk))) {
         case 8: if constexpr (NT % 8 == 0) return launch_column_tpl<OPT, NT, 8, FAST>(d, sc, f, ts, l, TW, Gs, counters, bad, s, mixed, walk, lanes.walk); break;
         case 4: if constexpr (NT % 4 == 0) return launch_column_tpl<OPT, NT, 4, FAST>(d, sc, f, ts, l, TW, Gs, counters, bad, s, mixed, walk, lanes.walk); break;
         case 2: if constexpr (NT % 2 == 0) return launch_column_tpl<OPT, NT, 2, FAST>(d, sc, f, ts, l, TW, Gs, counters, bad, s, mixed, walk, lanes.walk); break;

@@ -38,6 +38,7 @@
 // in the reference.
 #pragma once
 
+#include <algorithm>
 #include <type_traits>
 
 #include "face.h"
@@ -3246,20 +3247,30 @@ static inline long quad_lds(const Dims &d) {
     return (long)((d.wKUB - d.KLB) / 4 + 1) * 64 * (long)sizeof(double2);
 }
 
-// Where the quad walk is taken: while the lane per line leaves the 1,024 SIMDs
-// less than a wave (optimised path: its lane walk has the loads a level ahead)
-// or a wave and a half (the other path) each, and W and G of a column fit
-// 64 KB.  Measured with one tracer, lane walk -> quad walk: optimised path,
-// ragged columns, 28,000 / 44,000 / 63,000 lines of 40 levels 62 -> 42,
-// 65 -> 59, 79 -> 83 us; other path, 40 full levels, 40,000 / 90,000 / 122,000
-// lines 132 -> 65, 167 -> 125, 176 -> 185 us.
+// Where the quad walk is taken: while the lane per line leaves the 1,024 SIMDs few
+// waves each, and W and G of a column fit 64 KB.  Shallow columns give the four
+// lanes less of a chain to shorten, so the line moves with the levels; on the
+// optimised path, whose lane walk has the loads a level ahead, the quads also lose
+// once the LDS of the 256 CUs no longer holds all lines at a time (16 a block of
+// quad_lds bytes).  Measured, lane walk -> quad walk in us of the kernel, full columns:
+//   optimised path (2 tracers), 8 levels 16k lines 15 -> 13, 28k 15 -> 15, 40k 15 ->
+//     19; 20 levels 28k 30 -> 27, 40k 31 -> 32; 31 levels 40k 47 -> 42, 47k 47 -> 47;
+//     40 levels 44k 60 -> 54, 63k 61 -> 81; 60 levels 28k 88 -> 58, 40k 88 -> 96;
+//   other path (1 tracer), 8 levels 47k 24 -> 23, 63k 24 -> 26; 20 levels 63k 53 ->
+//     48, 78k 60 -> 63; 31 levels 95k 116 -> 93; 40 levels 122k 161 -> 151, 160k
+//     183 -> 209; 60 levels 95k 236 -> 211, 122k 247 -> 269.
+// A drop-in call counts the whole plane's columns, land included (its list's
+// length stays on the device).
 // form: MGPU_WALK_LANES keeps the lane walk, MGPU_WALK_QUADS the quad walk
 // wherever a column fits.
 template <bool OPT>
 static inline bool quad_columns(const Dims &d, long lines, int form) {
-    return quad_lds(d) <= 65536 &&
-           (form == MGPU_WALK_QUADS ||
-            (form == MGPU_WALK_AUTO && lines <= (OPT ? 48L : 96L) * 1024));
+    const long nk = d.wKUB - d.wKLB + 1, lds = quad_lds(d);
+    const long resident = 160 * 1024 / lds * 4096;
+    const long line = OPT ? std::min((16 + nk) * 1024, resident / 10 * 9)
+                          : std::min(96L, 32 + 2 * nk) * 1024;
+    return lds <= 65536 &&
+           (form == MGPU_WALK_QUADS || (form == MGPU_WALK_AUTO && lines <= line));
 }
 
 template <bool OPT, int NT, int TPL, bool FAST>

@@ -1744,9 +1744,9 @@ static int enqueue_steps(mgpu_transport *t, int nsteps, int cur, int dir) {
     const Dims &d = t->d;
     hipStream_t s = t->stream;
     const SharedFields f = make_fields(t->hydro, t->der, t->geom);
-    // face conductances (AD:1421-1478) on stream q; the depth-ordered column
-    // walk computes the W faces' itself
-    auto prep = [&](bool sw, hipStream_t q) {
+    // face conductances (AD:1421-1478); the depth-ordered column walk computes
+    // the W faces' itself
+    auto prep = [&](bool sw) {
         const bool nf = !t->sc.optimize && t->hydro.have_nf;
         return launch_prep_faces(d, t->hydro.visc, t->hydro.diffv, t->hydro.Qx, t->hydro.Qy,
                                  t->hydro.Qz, t->geom.DUX, t->geom.DVY, t->geom.DZX,
@@ -1755,7 +1755,7 @@ static int enqueue_steps(mgpu_transport *t, int nsteps, int cur, int dir) {
                                  t->sc.optimize ? 0 : t->nulldif,
                                  nf ? t->hydro.nfu : nullptr, nf ? t->hydro.nfv : nullptr,
                                  nf ? t->hydro.nfw : nullptr, 1, sw ? 0 : 1, t->der.cu,
-                                 t->der.cv, t->der.cw, q);
+                                 t->der.cv, t->der.cw, s);
     };
     for (int st = 0; st < nsteps; ++st) {
         StepScalars sc = t->sc;
@@ -1795,7 +1795,7 @@ static int enqueue_steps(mgpu_transport *t, int nsteps, int cur, int dir) {
         // tracers and 0.5 of 5.2 in the fast mode at 60 levels.)
         int rc;
         if ((rc = mark(t))) return rc;
-        if (st == 0 && (rc = prep(slot_walk(L, sc, f), s))) return rc;
+        if (st == 0 && (rc = prep(slot_walk(L, sc, f)))) return rc;
         if ((rc = mark(t))) return rc;
         // first kernel(s) of every chunk, then the second kernel(s)
         for (int ph = 1; ph <= 2; ++ph) {

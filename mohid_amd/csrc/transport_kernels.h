@@ -1269,7 +1269,8 @@ __device__ __forceinline__ int wave_min(int v) {
 // E0 being VolumeVariation's diagonal (AD:3994-4001).
 //
 // This is the non-optimised path (ComputeAdvection1D_V2 faces, any method and
-// limiter, NoAdvFlux, nudging); the optimised path is cell_rhs_opt.
+// limiter; NoAdvFlux in the drop-in's implicit rows, whose explicit cells and
+// nudging are explicit_tile_kernel's); the optimised path is cell_rhs_opt.
 template <bool OPT, int TPL, bool FAST, int IMP>
 __device__ __forceinline__ void cell_row_lane(const Dims &d, const StepScalars &sc,
                                               const SharedFields &f, const TracerSet &ts,
@@ -1302,7 +1303,7 @@ __device__ __forceinline__ void cell_row_lane(const Dims &d, const StepScalars &
     // implicit direction the D (fu*/fv*) and E (eu*/ev*) coefficients
     double fu0[TPL], fu1[TPL], fv0[TPL], fv1[TPL];
     double eu0[TPL], eu1[TPL], ev0[TPL], ev1[TPL];
-    // NoAdvFlux (the drop-in's lane kernels): a U face whose XX coefficients
+    // NoAdvFlux (the drop-in's implicit rows): a U face whose XX coefficients
     // the reference has cleared carries no advective flux (AD:4434-4443)
     // (non-optimised path only: compiled out of the optimised instances)
     const bool xzf = !OPT && f.xzero;
@@ -1360,23 +1361,17 @@ __device__ __forceinline__ void cell_row_lane(const Dims &d, const StepScalars &
             TI = TI + wv1 * g;
         }
         const bool au = IMP != 0, av = IMP != 1;   // explicit directions
-        // with nudging the advective terms gather in AdvectionTi, from zero
-        // (AD:4154-4157, 4665-4668, 5043-5046)
-        const bool nud = IMP < 0 && !OPT && TPL == 1 && f.nadv;
-        double A = nud ? 0.0 : TI;
         if (FAST) {
-            if (au && cfu0) A = A + fu0[t] * dtv;
-            if (au && cfu1) A = A - fu1[t] * dtv;
-            if (av && cfv0) A = A + fv0[t] * dtv;
-            if (av && cfv1) A = A - fv1[t] * dtv;
+            if (au && cfu0) TI = TI + fu0[t] * dtv;
+            if (au && cfu1) TI = TI - fu1[t] * dtv;
+            if (av && cfv0) TI = TI + fv0[t] * dtv;
+            if (av && cfv1) TI = TI - fv1[t] * dtv;
         } else {
-            if (au && cfu0) A = A + xdiv(fu0[t] * dt, Rv);
-            if (au && cfu1) A = A - xdiv(fu1[t] * dt, Rv);
-            if (av && cfv0) A = A + xdiv(fv0[t] * dt, Rv);
-            if (av && cfv1) A = A - xdiv(fv1[t] * dt, Rv);
+            if (au && cfu0) TI = TI + xdiv(fu0[t] * dt, Rv);
+            if (au && cfu1) TI = TI - xdiv(fu1[t] * dt, Rv);
+            if (av && cfv0) TI = TI + xdiv(fv0[t] * dt, Rv);
+            if (av && cfv1) TI = TI - xdiv(fv1[t] * dt, Rv);
         }
-        if (nud) f.nadv[x * s + t] = A;
-        else TI = A;
         TIo[t] = TI;
         if constexpr (IMP >= 0) {
             const bool c0 = IMP == 0 ? cfu0 : cfv0, c1 = IMP == 0 ? cfu1 : cfv1;

@@ -38,6 +38,13 @@ __global__ void __launch_bounds__(256) copy_set_kernel(CopySet c) {
 }  // namespace
 
 bool on_device(const void *p, hipStream_t s) {
+    // a process that sees one device needs no look-up (0.4 us each, 22 arrays in a
+    // set_geometry and a set_hydro: 12 of 433 us of a small coupled step)
+    static const bool only = [] {
+        int n = 0;
+        return hipGetDeviceCount(&n) == hipSuccess && n == 1;
+    }();
+    if (only) return true;
     int dev = 0;
     hipPointerAttribute_t a;
     if (hipStreamGetDevice(s, &dev) == hipSuccess && hipPointerGetAttributes(&a, p) == hipSuccess)

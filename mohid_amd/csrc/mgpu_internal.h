@@ -386,8 +386,8 @@ int launch_to_state(const Dims &d, const double *src, double *cur, double *other
 // Slot t of an interleaved buffer into a Fortran array.
 int launch_from_state(long n3, const double *src, double *dst, long stride, int t,
                       hipStream_t s);
-// Whether p is memory of stream s's own device: what its kernels may read and
-// write in place.
+// Whether the device pointer p is memory of stream s's own device: what its
+// kernels may read and write in place.
 bool on_device(const void *p, hipStream_t s);
 // Device arrays copied by one launch (a launch each leaves the copies of
 // arrays of some tens of MB at 2.2 TB/s; together they reach the card's);

@@ -24,6 +24,7 @@ static CopySet got;
 static dim3 grid, block;                               // of the launch under way
 
 extern "C" {
+hipError_t hipGetDeviceCount(int *n) { *n = 2; return hipSuccess; }
 hipError_t hipStreamGetDevice(hipStream_t, hipDevice_t *dev) { *dev = 0; return hipSuccess; }
 hipError_t hipPointerGetAttributes(hipPointerAttribute_t *a, const void *p) {
     const char *c = (const char *)p;
